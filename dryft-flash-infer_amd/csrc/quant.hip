@@ -12,6 +12,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <type_traits>
+
 #include "common.h"
 #include "../../include/qlinear.h"
 
@@ -32,81 +34,202 @@ int hip_status(hipError_t e, const char* what) {
   return QLX_EHIP;
 }
 
-// Natural column held at permuted position p of a 64-wide block (cuda_fp8.py:1117-1124):
-// p = 16t + 4s + i holds 16s + 2t + (0,1,8,9)[i].
-__device__ __forceinline__ int ref_natural(int p) {
-  const int t = p >> 4, s = (p >> 2) & 3, i = p & 3;
-  return 16 * s + 2 * t + ((i & 1) | ((i >> 1) << 3));
+// ---- weight quantize -----------------------------------------------------------------------
+
+// Largest magnitude of 8 bf16 values (pairs in v), ignoring NaNs.
+__device__ __forceinline__ float octet_amax(uint4 v, float amax) {
+  const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    amax = fmaxf(amax, fabsf(bf2f(d[j] & 0xffffu)));
+    amax = fmaxf(amax, fabsf(bf2f(d[j] >> 16)));
+  }
+  return amax;
 }
 
-// ---- weight quantize (one wave per (row, group)) ------------------------------------------
-
-// storage: 0 = offset bytes (q + offset, uint8, one per byte), 1 = signed int8,
-// 2 = int4 codes (q + 8) packed eight per int32 along K (nibble i of word j is k = 8j + i).
-__global__ void __launch_bounds__(256)
-quantize_weight_kernel(const uint16_t* __restrict__ w, void* __restrict__ data,
-                       uint16_t* __restrict__ scale, int rows, int k, int group, int bits,
-                       int scale_fp16, int nudge, int storage) {
-  const int lane = threadIdx.x & 63;
-  const long long gid = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int groups = k / group;
-  if (gid >= (long long)rows * groups) return;
-  const int row = (int)(gid / groups), g = (int)(gid % groups);
-  const uint16_t* src = w + (size_t)row * k + (size_t)g * group;
-  const int octets = group >> 3;
-  float amax = 0.f;
-  for (int o = lane; o < octets; o += 64) {
-    const uint4 v = *reinterpret_cast<const uint4*>(src + 8 * o);
-    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      amax = fmaxf(amax, fabsf(bf2f(d[j] & 0xffffu)));
-      amax = fmaxf(amax, fabsf(bf2f(d[j] >> 16)));
+// Integer codes of a group. storage: 0 = offset bytes (q + offset, uint8, one per byte), 1 = signed
+// int8, 2 = int4 codes (q + 8) packed eight per int32 along K (nibble i of word j is k = 8j + i).
+struct IntQuant {
+  int bits, scale_fp16, nudge, storage;
+  struct Group {
+    float sval, y, limit, offset;  // the stored scale's value, its reciprocal
+    uint16_t sbits;
+    bool fast;
+  };
+  __device__ __forceinline__ Group group(float amax) const {
+    Group g;
+    g.limit = bits == 8 ? 127.f : 7.f;
+    g.offset = bits == 8 ? 128.f : 8.f;
+    float s = fmaxf(amax / g.limit, 1e-12f);
+    if (nudge) s = s * (1.0f + 0.0009765625f);
+    if (scale_fp16) {
+      g.sbits = f2h(s);
+      g.sval = h2f(g.sbits);
+    } else {
+      g.sbits = f2bf(s);
+      g.sval = bf2f(g.sbits);
     }
+    g.y = 1.f / g.sval;
+    g.fast = g.sval >= 1e-30f && g.sval <= 3.40282347e38f;
+    return g;
   }
-  amax = wave_max(amax);
-  const float limit = bits == 8 ? 127.f : 7.f;
-  const float offset = bits == 8 ? 128.f : 8.f;
-  float s = fmaxf(amax / limit, 1e-12f);
-  if (nudge) s = s * (1.0f + 0.0009765625f);
-  uint16_t sbits;
-  float sval;
-  if (scale_fp16) {
-    sbits = f2h(s);
-    sval = h2f(sbits);
-  } else {
-    sbits = f2bf(s);
-    sval = bf2f(sbits);
-  }
-  if (lane == 0) scale[(size_t)row * groups + g] = sbits;
-  for (int o = lane; o < octets; o += 64) {
-    const uint4 v = *reinterpret_cast<const uint4*>(src + 8 * o);
+  // 8 values at element `at` of the flat weight. The quotient of the fast path is the IEEE one
+  // (quotient_by_reciprocal) wherever it can reach a code other than 0: a residual too small to
+  // be exact needs |x / s| far below 1/2. A zero or infinite scale and a chunk with a NaN divide.
+  __device__ __forceinline__ void store(const Group& g, uint4 v, void* data, size_t at) const {
     const uint32_t d[4] = {v.x, v.y, v.z, v.w};
     uint32_t codes[8];
+    if (g.fast && !(bf16_nan_bits(d[0]) | bf16_nan_bits(d[1]) | bf16_nan_bits(d[2]) | bf16_nan_bits(d[3]))) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float x = bf2f(e & 1 ? d[e >> 1] >> 16 : d[e >> 1] & 0xffffu);
-      float q = clamp_keep_nan(rintf(x / sval), limit);
-      if (storage == 1) {
-        codes[e] = q != q ? 0u : (uint32_t)(int32_t)q & 0xffu;
-      } else {
-        const float b = q + offset;
-        codes[e] = b != b ? 0u : (uint32_t)b;
+      for (int e = 0; e < 8; ++e) {
+        const float x = bf2f(e & 1 ? d[e >> 1] >> 16 : d[e >> 1] & 0xffffu);
+        const float q = __builtin_amdgcn_fmed3f(rintf(quotient_by_reciprocal(x, g.sval, g.y)), -g.limit, g.limit);
+        codes[e] = storage == 1 ? (uint32_t)(int32_t)q & 0xffu : (uint32_t)(q + g.offset);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = bf2f(e & 1 ? d[e >> 1] >> 16 : d[e >> 1] & 0xffffu);
+        float q = clamp_keep_nan(rintf(x / g.sval), g.limit);
+        if (storage == 1) {
+          codes[e] = q != q ? 0u : (uint32_t)(int32_t)q & 0xffu;
+        } else {
+          const float b = q + g.offset;
+          codes[e] = b != b ? 0u : (uint32_t)b;
+        }
       }
     }
-    const size_t kk = (size_t)g * group + 8 * o;
     if (storage == 2) {
       uint32_t word = 0;
 #pragma unroll
       for (int e = 0; e < 8; ++e) word |= (codes[e] & 0xfu) << (4 * e);
-      reinterpret_cast<uint32_t*>(data)[((size_t)row * k + kk) >> 3] = word;
+      reinterpret_cast<uint32_t*>(data)[at >> 3] = word;
     } else {
       uint2 out;
       out.x = codes[0] | (codes[1] << 8) | (codes[2] << 16) | (codes[3] << 24);
       out.y = codes[4] | (codes[5] << 8) | (codes[6] << 16) | (codes[7] << 24);
-      *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(data) + (size_t)row * k + kk) = out;
+      *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(data) + at) = out;
     }
   }
+};
+
+// e4m3 codes of a group (fp8.py:20-28): s = max(amax/448, 1e-12); code = e4m3(clamp(w/s)); scale
+// out bf16(s).
+struct Fp8Quant {
+  struct Group {
+    float sval, y;
+    uint16_t sbits;
+  };
+  __device__ __forceinline__ Group group(float amax) const {
+    const float s = fmaxf(amax / 448.f, 1e-12f);
+    return Group{s, 1.f / s, f2bf(s)};
+  }
+  __device__ __forceinline__ void store(const Group& g, uint4 v, void* data, size_t at) const {
+    *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(data) + at) = e4m3_chunk(v, g.sval, g.y);
+  }
+};
+
+// A row's groups follow each other, so group `gid` of the weight is the flat values
+// gid * group .. + group, and its scale the flat scale gid.
+//
+// Memory-bound (2 bytes in, 1/2 or 1 byte out per value) once every lane holds values and a value
+// costs about ten instructions: one wave per 128-value group left 48 of 64 lanes idle and divided
+// (IEEE division, ~30 instructions a value, and the values read twice): 151936 x 2560 to int4 in
+// 1362 us, 0.7 TB/s. Groups of up to 512 values: L lanes (8 values each) per group, 4 groups per
+// thread loaded before any is reduced: the same weight in 221 us, 4.4 TB/s (a large copy: 4.9 TB/s).
+constexpr int kSegs = 4;
+template <class Q, int L>
+__global__ void __launch_bounds__(256)
+quantize_segments_kernel(Q quant, const uint16_t* __restrict__ w, void* __restrict__ data,
+                         uint16_t* __restrict__ scale, long long segs, int group) {
+  const int lane = threadIdx.x % L, octets = group >> 3;
+  constexpr int PER = 256 / L;
+  const long long seg0 = (long long)blockIdx.x * (PER * kSegs) + threadIdx.x / L;
+  uint4 v[kSegs];
+#pragma unroll
+  for (int u = 0; u < kSegs; ++u) {
+    const long long seg = seg0 + u * PER;
+    v[u] = uint4{0u, 0u, 0u, 0u};
+    if (seg < segs && lane < octets) v[u] = *reinterpret_cast<const uint4*>(w + (size_t)seg * group + 8 * lane);
+  }
+#pragma unroll
+  for (int u = 0; u < kSegs; ++u) {
+    const long long seg = seg0 + u * PER;
+    float amax = octet_amax(v[u], 0.f);
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    if (seg >= segs) continue;
+    const typename Q::Group g = quant.group(amax);
+    if (lane == 0) scale[seg] = g.sbits;
+    if (lane < octets) quant.store(g, v[u], data, (size_t)seg * group + 8 * lane);
+  }
+}
+
+// Groups of 513 to 256 * 8 * R values (a row per scale): a 256-thread block per group, which keeps
+// its values in registers between the maximum and the codes.
+template <class Q, int R>
+__global__ void __launch_bounds__(256)
+quantize_rows_kernel(Q quant, const uint16_t* __restrict__ w, void* __restrict__ data,
+                     uint16_t* __restrict__ scale, int group) {
+  __shared__ float part[4];
+  const int octets = group >> 3;
+  const size_t base = (size_t)blockIdx.x * group;
+  uint4 v[R];
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int o = threadIdx.x + 256 * u;
+    v[u] = uint4{0u, 0u, 0u, 0u};
+    if (o < octets) v[u] = *reinterpret_cast<const uint4*>(w + base + 8 * o);
+  }
+  float amax = 0.f;
+#pragma unroll
+  for (int u = 0; u < R; ++u) amax = octet_amax(v[u], amax);
+  amax = wave_max(amax);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = amax;
+  __syncthreads();
+  amax = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+  const typename Q::Group g = quant.group(amax);
+  if (threadIdx.x == 0) scale[blockIdx.x] = g.sbits;
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const int o = threadIdx.x + 256 * u;
+    if (o < octets) quant.store(g, v[u], data, base + 8 * o);
+  }
+}
+
+// Longer groups: one wave per group, which reads the values twice.
+template <class Q>
+__global__ void __launch_bounds__(256)
+quantize_wave_kernel(Q quant, const uint16_t* __restrict__ w, void* __restrict__ data,
+                     uint16_t* __restrict__ scale, long long segs, int group) {
+  const int lane = threadIdx.x & 63, octets = group >> 3;
+  const long long seg = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (seg >= segs) return;
+  const uint16_t* src = w + (size_t)seg * group;
+  float amax = 0.f;
+  for (int o = lane; o < octets; o += 64) amax = octet_amax(*reinterpret_cast<const uint4*>(src + 8 * o), amax);
+  const typename Q::Group g = quant.group(wave_max(amax));
+  if (lane == 0) scale[seg] = g.sbits;
+  for (int o = lane; o < octets; o += 64)
+    quant.store(g, *reinterpret_cast<const uint4*>(src + 8 * o), data, (size_t)seg * group + 8 * o);
+}
+
+template <class Q>
+void launch_quantize(const Q& quant, const uint16_t* w, void* data, uint16_t* scale, int rows, int k, int group,
+                     hipStream_t st) {
+  const long long segs = (long long)rows * (k / group);
+  const int octets = group >> 3;
+  auto segments = [&](auto lc) {
+    constexpr int L = decltype(lc)::value, per = 256 / L * kSegs;
+    quantize_segments_kernel<Q, L><<<(unsigned)((segs + per - 1) / per), 256, 0, st>>>(quant, w, data, scale, segs, group);
+  };
+  if (octets <= 8) segments(std::integral_constant<int, 8>{});
+  else if (octets <= 16) segments(std::integral_constant<int, 16>{});
+  else if (octets <= 32) segments(std::integral_constant<int, 32>{});
+  else if (octets <= 64) segments(std::integral_constant<int, 64>{});
+  else if (octets <= 512) quantize_rows_kernel<Q, 2><<<(unsigned)segs, 256, 0, st>>>(quant, w, data, scale, group);
+  else if (octets <= 2048) quantize_rows_kernel<Q, 8><<<(unsigned)segs, 256, 0, st>>>(quant, w, data, scale, group);
+  else quantize_wave_kernel<Q><<<(unsigned)((segs + 3) / 4), 256, 0, st>>>(quant, w, data, scale, segs, group);
 }
 
 // ---- dequantize: bf16((q - offset) * float(scale)) -------------------------------------
@@ -135,46 +258,58 @@ dequantize_kernel(const void* __restrict__ data, const uint16_t* __restrict__ sc
 
 // ---- reference layouts (cuda_fp8.Prepared) --------------------------------------------------
 
-// Output byte o of the prepared weight, gathered from the [rows, K] quantize output.
+// The prepared weight from the [rows, K] quantize output: a thread takes one 64-value block of one
+// row (4 bits: the two blocks of a 128-value step) and writes the 64 bytes it becomes, which every
+// layout keeps together: position 16t + 4s + i of a permuted block holds the natural value
+// 16s + 2t + (0, 1, 8, 9)[i] (cuda_fp8.py:1117-1124), so dword s of the 16 bytes of t is the value
+// pairs 16s + 2t and 16s + 2t + 8. (It gathered single bytes, each through six 64-bit divisions.)
+// The bytes may start anywhere (a slice of a larger buffer): accesses are declared unaligned.
+struct __attribute__((packed, aligned(1))) Bytes16 {
+  uint32_t x, y, z, w;
+};
 __global__ void __launch_bounds__(256)
 prepare_ref_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int rows,
                    int k, int bits, int tiled) {
   const size_t o = (size_t)blockIdx.x * 256 + threadIdx.x;
-  const int width = bits == 4 ? k / 2 : k;
-  if (o >= (size_t)rows * width) return;
-  if (!tiled) {  // 8-bit row-major, fragment-permuted columns
-    const int r = (int)(o / k), pos = (int)(o % k);
-    dst[o] = src[(size_t)r * k + (pos & ~63) + ref_natural(pos & 63)];
-    return;
-  }
-  const int groups = k / 128;
+  const int per_row = k >> (bits == 4 ? 7 : 6);
+  if (o >= (size_t)rows * per_row) return;
+  const int r = (int)(o / per_row), blk = (int)(o - (size_t)r * per_row);
+  auto block = [&](int b64, uint32_t (&out)[16]) {  // 64 values, permuted
+    const Bytes16* p = reinterpret_cast<const Bytes16*>(src + (size_t)r * k + (size_t)b64 * 64);
+    uint32_t d[16];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const Bytes16 v = p[i];
+      d[4 * i] = v.x, d[4 * i + 1] = v.y, d[4 * i + 2] = v.z, d[4 * i + 3] = v.w;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        out[4 * t + s] = __builtin_amdgcn_perm(d[4 * s + 2 + (t >> 1)], d[4 * s + (t >> 1)],
+                                               t & 1 ? 0x07060302u : 0x05040100u);
+  };
+  uint32_t out[16];
+  size_t at;
+  const size_t tile = r >> 4;
+  const int half = (r >> 3) & 1, gg = r & 7;
   if (bits == 8) {
-    // (tile, group, half, j, g, t, byte) = 16 * 2048-byte tiles per row block
-    size_t rest = o;
-    const int byte = rest % 16; rest /= 16;
-    const int t = rest % 4; rest /= 4;
-    const int gg = rest % 8; rest /= 8;
-    const int j = rest % 2; rest /= 2;
-    const int half = rest % 2; rest /= 2;
-    const int grp = rest % groups; rest /= groups;
-    const int tile = (int)rest;
-    const int row = tile * 16 + half * 8 + gg;
-    const int pos = j * 64 + t * 16 + byte;
-    dst[o] = src[(size_t)row * k + grp * 128 + (pos & ~63) + ref_natural(pos & 63)];
+    block(blk, out);
+    // tiled: [tile][K/128][half][j][g][t][16 B]
+    at = tiled ? ((((tile * (k >> 7) + (blk >> 1)) * 2 + half) * 2 + (blk & 1)) * 8 + gg) * 64
+               : (size_t)r * k + (size_t)blk * 64;
   } else {
-    // (tile, group, half, g, t, byte); block 0 in the low nibble, block 1 in the high one
-    size_t rest = o;
-    const int byte = rest % 16; rest /= 16;
-    const int t = rest % 4; rest /= 4;
-    const int gg = rest % 8; rest /= 8;
-    const int half = rest % 2; rest /= 2;
-    const int grp = rest % groups; rest /= groups;
-    const int tile = (int)rest;
-    const int row = tile * 16 + half * 8 + gg;
-    const size_t base = (size_t)row * k + grp * 128;
-    const int nat = ref_natural(t * 16 + byte);
-    dst[o] = (uint8_t)((src[base + nat] & 0xf) | ((src[base + 64 + nat] & 0xf) << 4));
+    // [tile][K/128][half][g][t][16 B]; block 0 in the low nibble, block 1 in the high one
+    uint32_t hi[16];
+    block(2 * blk, out);
+    block(2 * blk + 1, hi);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) out[i] = (out[i] & 0x0f0f0f0fu) | ((hi[i] & 0x0f0f0f0fu) << 4);
+    at = (((tile * (k >> 7) + blk) * 2 + half) * 8 + gg) * 64;
   }
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    reinterpret_cast<Bytes16*>(dst + at)[i] = Bytes16{out[4 * i], out[4 * i + 1], out[4 * i + 2], out[4 * i + 3]};
 }
 
 // Tiled 8-bit prepared weight -> fragment-permuted row-major bytes.
@@ -191,35 +326,6 @@ row_major_ref_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
 }
 
 // ---- FP8 e4m3 (fp8.py:20-28) ------------------------------------------------------------------
-
-// One wave per (row, group): s = max(amax/448, 1e-12); code = e4m3(clamp(w/s)); scale out bf16(s).
-__global__ void __launch_bounds__(256)
-quantize_fp8_weight_kernel(const uint16_t* __restrict__ w, uint8_t* __restrict__ code,
-                           uint16_t* __restrict__ scale, int rows, int k, int group) {
-  const int lane = threadIdx.x & 63;
-  const long long gid = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int groups = k / group;
-  if (gid >= (long long)rows * groups) return;
-  const int row = (int)(gid / groups), g = (int)(gid % groups);
-  const uint16_t* src = w + (size_t)row * k + (size_t)g * group;
-  uint8_t* dst = code + (size_t)row * k + (size_t)g * group;
-  const int octets = group >> 3;
-  float amax = 0.f;
-  for (int o = lane; o < octets; o += 64) {
-    const uint4 v = *reinterpret_cast<const uint4*>(src + 8 * o);
-    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      amax = fmaxf(amax, fabsf(bf2f(d[j] & 0xffffu)));
-      amax = fmaxf(amax, fabsf(bf2f(d[j] >> 16)));
-    }
-  }
-  amax = wave_max(amax);
-  const float s = fmaxf(amax / 448.f, 1e-12f), y = 1.f / s;
-  if (lane == 0) scale[(size_t)row * groups + g] = f2bf(s);
-  for (int o = lane; o < octets; o += 64)
-    *reinterpret_cast<uint2*>(dst + 8 * o) = e4m3_chunk(*reinterpret_cast<const uint4*>(src + 8 * o), s, y);
-}
 
 // Per-token activation quantize: one block of 256 threads per row.
 __global__ void __launch_bounds__(256)
@@ -355,10 +461,8 @@ int qlx_quantize_weight(const void* w, void* data, void* scale, int rows, int k,
   QLX_REQUIRE(storage != 2 || bits == 4, "int4 k32 packing needs bits=4");
   QLX_REQUIRE(storage != 1 || bits == 8, "signed storage needs bits=8");
   QLX_REQUIRE(scale_kind == QLX_SCALE_F16 || scale_kind == QLX_SCALE_BF16, "bad scale kind");
-  const size_t work = (size_t)rows * (k / group);
-  quantize_weight_kernel<<<blocks_for(work, 4), 256, 0, (hipStream_t)stream>>>(
-      (const uint16_t*)w, data, (uint16_t*)scale, rows, k, group, bits,
-      scale_kind == QLX_SCALE_F16, nudge, storage);
+  launch_quantize(IntQuant{bits, scale_kind == QLX_SCALE_F16, nudge, storage}, (const uint16_t*)w, data,
+                  (uint16_t*)scale, rows, k, group, (hipStream_t)stream);
   QLX_LAUNCH_CHECK("quantize_weight");
 }
 
@@ -377,7 +481,7 @@ int qlx_prepare_ref(const void* data, void* out, int rows, int k, int bits, int 
   QLX_REQUIRE(rows % 16 == 0, "rows=%d is not a multiple of 16", rows);
   QLX_REQUIRE(bits == 8 || bits == 4, "weights are 8 or 4 bits");
   QLX_REQUIRE(bits == 8 || tiled, "4-bit weights are stored tiled");
-  const size_t n = (size_t)rows * (bits == 4 ? k / 2 : k);
+  const size_t n = (size_t)rows * (k / (bits == 4 ? 128 : 64));
   prepare_ref_kernel<<<blocks_for(n, 256), 256, 0, (hipStream_t)stream>>>(
       (const uint8_t*)data, (uint8_t*)out, rows, k, bits, tiled);
   QLX_LAUNCH_CHECK("prepare_ref");
@@ -394,9 +498,7 @@ int qlx_quantize_fp8_weight(const void* w, void* code, void* scale, int rows, in
                             void* stream) {
   QLX_REQUIRE(rows > 0 && k > 0 && group > 0 && k % group == 0, "%d is not a multiple of %d", k, group);
   QLX_REQUIRE(group % 8 == 0, "group %d must be a multiple of 8", group);
-  const size_t work = (size_t)rows * (k / group);
-  quantize_fp8_weight_kernel<<<blocks_for(work, 4), 256, 0, (hipStream_t)stream>>>(
-      (const uint16_t*)w, (uint8_t*)code, (uint16_t*)scale, rows, k, group);
+  launch_quantize(Fp8Quant{}, (const uint16_t*)w, code, (uint16_t*)scale, rows, k, group, (hipStream_t)stream);
   QLX_LAUNCH_CHECK("quantize_fp8_weight");
 }
 
