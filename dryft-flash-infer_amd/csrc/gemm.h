@@ -31,6 +31,8 @@
 // the same MFMA chain with the codes all at the bias, so zero weights cancel exactly.
 #pragma once
 
+#include <type_traits>
+
 #include "common.h"
 #include "../../include/qlinear.h"
 
@@ -162,6 +164,15 @@ __device__ __forceinline__ void settle_batch(const GemmArgs& a, const XS& xs, ty
       for (int u = 0; u < U; ++u)
         if ((stale >> u & 1u) && xs.ready(r[u])) stale &= ~(1u << u);
     }
+  }
+}
+
+// fn(integral_constant<int, P>) for P = B .. E - 1, unrolled at compile time.
+template <int B, int E, class Fn>
+__host__ __device__ __forceinline__ void static_for(Fn&& fn) {
+  if constexpr (B < E) {
+    fn(std::integral_constant<int, B>{});
+    static_for<B + 1, E>(fn);
   }
 }
 
@@ -1189,10 +1200,13 @@ __device__ __forceinline__ void add_norm_ticket(const GemmArgs& a) {
   add_norm_tail(a);
 }
 
-// y = bf16(bf16(silu(g)) * u) with g and u rounded to bf16 first (swiglu.py:12-30).
+// y = bf16(bf16(silu(g)) * u) with g and u rounded to bf16 first (swiglu.py:12-30); the caller rounds
+// the product. The roundings are the hardware's pair conversion (a NaN stays a NaN).
 __device__ __forceinline__ float swiglu_bf(float g, float u) {
-  const float gb = round_bf(g), ub = round_bf(u);
-  return round_bf(gb / (1.f + expf(-gb))) * ub;
+  const uint32_t gu = bf16_pair_hw(g, u);
+  const float gb = bf2f(gu & 0xffffu);
+  const float s = gb / (1.f + expf(-gb));
+  return bf2f(bf16_pair_hw(s, s) & 0xffffu) * __uint_as_float(gu & 0xffff0000u);
 }
 
 // Stage the activation (from xs), then stream the item's weight steps through the MFMAs into

@@ -273,15 +273,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t skinny_rsrc(const void* p, uns
 // Buffer access policy sc1: device scope (past this XCD's L2, which other XCDs' stores do not update).
 constexpr int kSc1 = 16;
 
-// fn(integral_constant<int, P>) for P = B .. E - 1, unrolled at compile time.
-template <int B, int E, class Fn>
-__device__ __forceinline__ void static_for(Fn&& fn) {
-  if constexpr (B < E) {
-    fn(std::integral_constant<int, B>{});
-    static_for<B + 1, E>(fn);
-  }
-}
-
 // Two workgroups per CU (each wave at most 256 registers), or one for the wide instances.
 template <class F, int MT, int RW, int WAVES, bool SW>
 __global__ void __launch_bounds__(WAVES * 64)

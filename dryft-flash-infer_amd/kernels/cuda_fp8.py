@@ -27,7 +27,7 @@ The same signatures also carry the MI355X north-star formats, so an engine that 
   ``FormatPrepared`` with the attributes the engine reads (``bits``, ``k``, ``rows``,
   ``bytes_moved()``);
 * the linears dispatch on it: ``matmul``/``gate_up_swiglu`` take the library's planned
-  path for the batch (decode kernel, skinny GEMM from 9 tokens, FP8 activation quantized
+  path for the batch (the resident-activation GEMM where its plan has the call, else decode kernel or skinny GEMM; FP8 activation quantized
   once from 2 tokens), ``matmul_partials``/``splits`` honour the config's split-K.
 """
 
@@ -247,6 +247,29 @@ def _fmt(prepared):
     return _lib.FMT_REF8 if prepared.bits == 8 else _lib.FMT_REF4
 
 
+def _resident_plan(prepared, batch, config, mode):
+    """The resident GEMM's plan (``qlx_linear_resident``) for a call on tiled reference-format weights,
+    or None: a config that asks for K slices gets them from the decode kernel, whose planes sum to
+    its result. A config of one slice leaves the slices to the library: where the decode kernel
+    would cut K to fit its LDS, the planes are the resident GEMM's too."""
+    if prepared.fmt != "ref" or not prepared.tiled or batch > 64:
+        return None
+    if mode != _lib.MODE_SWIGLU and _splitk(prepared, config) > 1:
+        return None
+    fmt = _fmt(prepared)
+    if mode == _lib.MODE_PLANES:
+        cfg = _plan_config(prepared, batch, config, mode)
+        if _linear.splits_for(fmt, mode, batch, prepared.rows, prepared.k, cfg, fit=True) == 1:
+            return None
+    from . import qlinear
+    if not qlinear.aligned(prepared.weight, prepared.scale):
+        return None
+    plan = qlinear.plan_resident(fmt, batch, prepared.rows, prepared.k, mode == _lib.MODE_SWIGLU)
+    if plan is not None:
+        plan.mode = mode
+    return plan
+
+
 def _run(x, prepared, config, mode):
     batch, k = x.shape
     if k != prepared.k:
@@ -259,7 +282,12 @@ def _run(x, prepared, config, mode):
         linear = qlinear.FORMATS[prepared.fmt][1]
         if mode == _lib.MODE_PLANES:
             return linear(x, prepared.tiles, config=_plan_config(prepared, batch, config, mode), planes=True)
-        return linear(x, prepared.tiles, swiglu=mode == _lib.MODE_SWIGLU)
+        return linear(x, prepared.tiles, swiglu=mode == _lib.MODE_SWIGLU, resident=True)
+    plan = _resident_plan(prepared, batch, config, mode)
+    if plan is not None:
+        from . import qlinear
+        return qlinear.run_resident(plan, _fmt(prepared), prepared.weight, prepared.scale, x, None, batch,
+                                    prepared.rows, k)
     cfg = _plan_config(prepared, batch, config, mode)
     return _linear.run(_fmt(prepared), "qlx_linear_ref", x, prepared.rows, prepared.k,
                        (_lib.ptr(prepared.weight), _lib.ptr(prepared.scale), _lib.ptr(x)),
@@ -268,6 +296,9 @@ def _run(x, prepared, config, mode):
 
 def splits(prepared: Prepared, batch: int, config=(4, 1)) -> int:
     """How many fp32 planes ``matmul_partials`` returns for this shape and config."""
+    plan = _resident_plan(prepared, batch, config, _lib.MODE_PLANES)
+    if plan is not None:
+        return plan.splits
     cfg = _plan_config(prepared, batch, config, _lib.MODE_PLANES)
     return _linear.splits_for(_fmt(prepared), _lib.MODE_PLANES, batch, prepared.rows, prepared.k, cfg, fit=True)
 

@@ -51,13 +51,14 @@ class Candidate:
     bits: int = 16
 
 
-def north_matmul(x, operand, *, config=None, skinny=None, pre_quantize=None):
+def north_matmul(x, operand, *, config=None, skinny=None, pre_quantize=None, resident=None):
     """``x @ W^T`` for a north-star operand (``cuda_fp8.FormatPrepared`` or ``qlinear.Tiled``)
     on one chosen path: ``config`` a ``(waves, kw, rw, splits)`` plan of the decode kernel,
-    ``skinny`` the skinny GEMM, ``pre_quantize`` the FP8 activation's quantization placement."""
+    ``skinny`` the skinny GEMM, ``resident`` the resident-activation GEMM, ``pre_quantize`` the FP8
+    activation's quantization placement."""
     from . import qlinear
     tiles = getattr(operand, "tiles", operand)
-    kwargs = {"config": config}
+    kwargs = {"config": config, "resident": resident}
     if tiles.fmt == "fp8":
         kwargs["pre_quantize"] = pre_quantize
     else:
@@ -95,6 +96,7 @@ def _north_candidates(batch, packed, quick):
         lib_fmt = {"w8a16": _lib.FMT_W8A16, "w4a16": _lib.FMT_W4A16, "fp8": _lib.FMT_FP8}[fmt]
         plan = _linear.make_plan(lib_fmt, _lib.MODE_BF16, batch, tiles.rows, tiles.k)
         steps = tiles.k // (256 if fmt == "w4a16" else 128)
+        variants.append(("resident GEMM", {"resident": True}))
         for mul in (2, 4):
             if plan.splits * mul <= steps:
                 variants.append((f"decode split-K {plan.splits * mul}",

@@ -196,6 +196,55 @@ def _skinny(fmt, q, s, x, n, k, swiglu, fused_reduce=None):
     return out
 
 
+#: Up to this many tokens the resident-activation GEMM (``qlx_linear_resident``) is the default where
+#: its plan has the call; ``resident=True`` takes it at any batch. From 9 tokens these functions'
+#: default stays the skinny GEMM, whose bits callers compare with ``qlx_linear_skinny``'s; the
+#: engine's call sites (``cuda_fp8.matmul``, ``gate_up_swiglu``) pass ``resident=True``.
+RESIDENT_TO = 8
+
+
+def plan_resident(fmt, m, n, k, swiglu=False):
+    """The resident GEMM's plan for a call, or None where another kernel serves it."""
+    plan = _lib.Plan()
+    _lib.check(_lib.lib().qlx_plan_resident(fmt, _mode(swiglu), m, n, k, plan), "plan_resident")
+    return plan if plan.splits > 0 else None
+
+
+def run_resident(plan, fmt, q, s, x, xs, m, n, k):
+    """``qlx_linear_resident`` with ``plan``: bf16 ``[m, n]`` (SwiGLU ``[m, n/2]``), or fp32 planes
+    ``[splits, m, n]`` where the plan's mode is planes."""
+    device = x.device
+    planes = plan.mode == _lib.MODE_PLANES
+    work = out = None
+    if x.data_ptr() % 16:  # the kernel reads it in 16-byte pieces
+        x = x.clone()
+    if planes or plan.splits > 1:
+        work = torch.empty((plan.splits, m, n), dtype=torch.float32, device=device)
+        plan.workspace = work.data_ptr()
+    if not planes:
+        out = torch.empty((m, n // 2 if plan.mode == _lib.MODE_SWIGLU else n), dtype=torch.bfloat16, device=device)
+        if plan.splits > 1:
+            plan.tickets = _lib.tickets(device, 512).data_ptr()
+    _lib.call("qlx_linear_resident", fmt, _lib.ptr(q), _lib.ptr(s), _lib.ptr(x), _lib.ptr(xs), _lib.ptr(out), m, n, k,
+              ctypes.byref(plan), _lib.stream(device))
+    return work if planes else out
+
+
+def aligned(weight, scale):
+    """Whether a weight starts where the resident GEMM's buffer loads need it."""
+    return weight.data_ptr() % 16 == 0 and scale.data_ptr() % 4 == 0
+
+
+def _use_resident(resident, skinny, fmt, q, s, x, n, k, tiled, planes, config, swiglu):
+    """The plan of the resident GEMM if the call takes it: asked for, or by default up to
+    ``RESIDENT_TO`` tokens; tile-layout weights, the library's plan, aligned operands."""
+    if resident is None:
+        resident = skinny is None and x.shape[0] <= RESIDENT_TO
+    if not resident or skinny or not tiled or planes or config is not None or not aligned(q, s):
+        return None
+    return plan_resident(fmt, x.shape[0], n, k, swiglu)
+
+
 #: From this many tokens the skinny GEMM is the default (tile-layout W4A16/W8A16
 #: weights, library plan): at 16-64 tokens it is 1.5-7.5x faster than the decode kernel.
 SKINNY_FROM = 9
@@ -209,28 +258,35 @@ def _use_skinny(skinny, x, tiled, planes, config):
     return bool(skinny)
 
 
-def linear_w8a16(x, packed, config=None, planes=False, swiglu=False, skinny=None):
+def linear_w8a16(x, packed, config=None, planes=False, swiglu=False, skinny=None, resident=None):
     """``x @ deq(W).T`` for W8A16 per-channel weights; bf16 ``[M, N]`` (SwiGLU: ``[M, N/2]``).
     ``skinny`` (None: from 9 tokens on tile-layout weights) runs the skinny GEMM, whose
-    activation streams through LDS per K step; False forces the decode kernel."""
+    activation streams through LDS per K step; False forces the decode kernel. ``resident``
+    (None: up to 8 tokens) runs the resident-activation GEMM where its plan has the call."""
     q, s, n, k, tiled = _unpack(packed, "w8a16")
     _check_x(x, k)
     _lib.require_device(q, s)
     if s.numel() != n:
         raise ValueError("W8A16 scales are one bf16 per output channel")
+    plan = _use_resident(resident, skinny, _lib.FMT_W8A16, q, s, x, n, k, tiled, planes, config, swiglu)
+    if plan is not None:
+        return run_resident(plan, _lib.FMT_W8A16, q, s, x, None, x.shape[0], n, k)
     if _use_skinny(skinny, x, tiled, planes, config):
         return _skinny(_lib.FMT_W8A16, q, s, x, n, k, swiglu)
     return _linear.run(_lib.FMT_W8A16, "qlx_linear_w8a16", x, n, k,
                        (_lib.ptr(q), _lib.ptr(s), _lib.ptr(x)), (tiled,), mode=_mode(swiglu, planes), config=config)
 
 
-def linear_w4a16(x, packed, config=None, planes=False, swiglu=False, skinny=None):
-    """``x @ deq(W).T`` for W4A16 group-128 weights (``skinny``: as in ``linear_w8a16``)."""
+def linear_w4a16(x, packed, config=None, planes=False, swiglu=False, skinny=None, resident=None):
+    """``x @ deq(W).T`` for W4A16 group-128 weights (``skinny``, ``resident``: as in ``linear_w8a16``)."""
     q, s, n, k, tiled = _unpack(packed, "w4a16")
     _check_x(x, k)
     _lib.require_device(q, s)
     if q.dtype != torch.int32 or tuple(s.shape) != (n, k // 128):
         raise ValueError("W4A16 weights are int32 [N, K/8] with bf16 scales [N, K/128]")
+    plan = _use_resident(resident, skinny, _lib.FMT_W4A16, q, s, x, n, k, tiled, planes, config, swiglu)
+    if plan is not None:
+        return run_resident(plan, _lib.FMT_W4A16, q, s, x, None, x.shape[0], n, k)
     if _use_skinny(skinny, x, tiled, planes, config):
         return _skinny(_lib.FMT_W4A16, q, s, x, n, k, swiglu)
     return _linear.run(_lib.FMT_W4A16, "qlx_linear_w4a16", x, n, k,
@@ -263,11 +319,13 @@ def _skinny_fp8(q, s, xq, sx, n, k, swiglu, fused_reduce=None):
     return out
 
 
-def linear_fp8_w8a8(x, packed, config=None, planes=False, swiglu=False, pre_quantize=None, skinny=None):
+def linear_fp8_w8a8(x, packed, config=None, planes=False, swiglu=False, pre_quantize=None, skinny=None,
+                    resident=None):
     """``(x_q s_x) @ (W_q s_w).T`` with the activation quantized per token (``pre_quantize``:
     None = by its own kernel from 2 tokens, else inside the GEMM; the codes are the same).
     ``skinny`` (None: from 9 tokens on tile-layout weights) runs the skinny GEMM on the
-    quantized codes; False forces the decode kernel."""
+    quantized codes; False forces the decode kernel. ``resident``: as in ``linear_w8a16``, on codes
+    quantized beforehand."""
     q, s, n, k, tiled = _unpack(packed, "fp8")
     _check_x(x, k)
     _lib.require_device(q, s)
@@ -275,6 +333,10 @@ def linear_fp8_w8a8(x, packed, config=None, planes=False, swiglu=False, pre_quan
         raise ValueError("FP8 W8A8 weight scales are one bf16 per output channel")
     if skinny is None and pre_quantize is not None:  # a decode-kernel variant was asked for
         skinny = False
+    plan = _use_resident(resident, skinny, _lib.FMT_FP8, q, s, x, n, k, tiled, planes, config, swiglu)
+    if plan is not None:
+        xq, sx = quantize_fp8_activation(x)
+        return run_resident(plan, _lib.FMT_FP8, q, s, xq, sx, x.shape[0], n, k)
     if _use_skinny(skinny, x, tiled, planes, config):
         if pre_quantize is False:
             raise ValueError("the FP8 skinny GEMM takes the activation quantized beforehand")
@@ -291,10 +353,10 @@ def linear_fp8_w8a8(x, packed, config=None, planes=False, swiglu=False, pre_quan
                        (_lib.ptr(q), _lib.ptr(s), _lib.ptr(x)), (tiled,), mode=_mode(swiglu, planes), config=config)
 
 
-def linear_fp8_w8a8_quantized(xq, sx, packed, config=None, planes=False, swiglu=False, skinny=None):
+def linear_fp8_w8a8_quantized(xq, sx, packed, config=None, planes=False, swiglu=False, skinny=None, resident=None):
     """FP8 W8A8 linear of an activation quantized beforehand: e4m3 codes ``xq`` [m, k] with
     fp32 per-token scales ``sx`` [m] (``quantize_fp8_activation`` or ``add_norm_quant_fp8``).
-    ``skinny`` as for ``linear_fp8_w8a8``."""
+    ``skinny``, ``resident`` as for ``linear_fp8_w8a8``."""
     q, s, n, k, tiled = _unpack(packed, "fp8")
     if xq.ndim != 2 or xq.shape[1] != k or xq.element_size() != 1:
         raise ValueError("codes must be one byte each, [m, k] with k the weight's width")
@@ -303,6 +365,9 @@ def linear_fp8_w8a8_quantized(xq, sx, packed, config=None, planes=False, swiglu=
     if not 1 <= xq.shape[0] <= 64:
         raise ValueError(f"batch {xq.shape[0]} exceeds 64 rows")
     _lib.require_device(q, s, xq, sx)
+    plan = _use_resident(resident, skinny, _lib.FMT_FP8, q, s, xq, n, k, tiled, planes, config, swiglu)
+    if plan is not None:
+        return run_resident(plan, _lib.FMT_FP8, q, s, xq, sx, xq.shape[0], n, k)
     if _use_skinny(skinny, xq, tiled, planes, config):
         return _skinny_fp8(q, s, xq.view(torch.uint8), sx, n, k, swiglu)
     return _linear.run(_lib.FMT_FP8, "qlx_linear_fp8_w8a8_q", xq, n, k,

@@ -179,6 +179,19 @@ int qlx_linear_skinny(int fmt, const void* w, const void* w_scale, const void* x
 int qlx_linear_skinny_fp8(const void* w, const void* w_scale, const void* x_code, const float* x_scale, void* y,
                           int m, int n, int k, const qlx_plan* plan, void* stream);
 
+/* The resident-activation GEMM for 1..64 tokens, every tile-layout format (QLX_FMT_W4A16, W8A16,
+ * FP8, and the reference's tiled REF8 / REF4): each wave keeps its K range's activation fragments
+ * in registers for the whole launch and streams that range of a run of 16-row weight tiles. FP8
+ * takes the activation quantized beforehand (e4m3 codes, x_scale fp32 [m]); the others bf16 x and
+ * no x_scale. Output bf16, SwiGLU, or the fp32 planes themselves (QLX_MODE_PLANES, in plan->workspace,
+ * y unused); weights of under 2 GiB; w and x on 16-byte boundaries. qlx_plan_resident
+ * fills plan->splits: 0 where no slice count fits the registers or another kernel measured faster
+ * (qlx_linear_* / qlx_linear_skinny* serve those calls). With splits > 1 the call takes a workspace
+ * of splits * m * n floats and 512 zeroed tickets (zero again afterwards). */
+int qlx_plan_resident(int fmt, int mode, int m, int n, int k, qlx_plan* plan);
+int qlx_linear_resident(int fmt, const void* w, const void* w_scale, const void* x, const float* x_scale, void* y,
+                        int m, int n, int k, const qlx_plan* plan, void* stream);
+
 /* qlx_linear_skinny for callers that cannot allocate (code under graph capture, serving
  * loops, harnesses that forbid hipMalloc): no counterpart in the reference. It plans the call
  * itself (qlx_plan_skinny) and keeps the K-slice planes and ticket counters in the library's
