@@ -53,6 +53,14 @@ __device__ __forceinline__ uint32_t bf16_pair_hw(float lo, float hi) {
 // Bits 15 / 31 set where the low / high bf16 half of p is a NaN.
 __device__ __forceinline__ uint32_t bf16_nan_bits(uint32_t p) { return ((p & 0x7fff7fffu) + 0x007f007fu) & 0x80008000u; }
 
+// The NaN halves of p (a pair of bf16_pair_hw) in the form f2bf gives them, sign | 0x7FC0: the hardware
+// keeps a NaN's sign, so rounding a chain of values by pairs and passing its results through here gives
+// f2bf's bits, with no second copy of the chain's code.
+__device__ __forceinline__ uint32_t bf16_canonical_nan(uint32_t p) {
+  const uint32_t m = (bf16_nan_bits(p) >> 15) * 0xffffu;
+  return (p & ~m) | (m & ((p & 0x80008000u) | 0x7fc07fc0u));
+}
+
 __device__ __forceinline__ float h2f(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 
 // fp32 -> fp16 bits, RNE (hardware v_cvt_f16_f32 rounds to nearest even).

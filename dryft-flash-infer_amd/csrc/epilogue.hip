@@ -14,6 +14,8 @@
 
 namespace qlx {
 
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+
 __global__ void __launch_bounds__(256)
 reduce_planes_kernel(const float* __restrict__ p, uint16_t* __restrict__ out, size_t width, int splits) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -33,227 +35,238 @@ residual_planes_kernel(const uint16_t* __restrict__ x, const float* __restrict__
   out[i] = f2bf(bf2f(x[i]) + round_bf(acc));
 }
 
-// Chunks of 8 values a thread of add_rms_norm_kernel loads at once (n <= 256 * 8 * 8 = 16384).
-constexpr int kNormChunks = 8;
-
 __device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
   return (uint32_t)f2bf(lo) | ((uint32_t)f2bf(hi) << 16);
 }
 
 __device__ __forceinline__ uint4 ld16(const uint16_t* p) {
-  const u32x4 v = *reinterpret_cast<const u32x4*>(p);
+  const u32x4 v = *gmem(reinterpret_cast<const u32x4*>(p));
   return uint4{v[0], v[1], v[2], v[3]};
 }
 
-// delta: bf16 [rows][n] or (planes != null) fp32 planes [splits][rows][n]; res may be null
-// (plain rms_norm of x). One workgroup of 256 threads per row. When n % 8 == 0 every thread
-// issues all of its 16-byte loads (x, delta or each plane, w) before it uses any, so a row
-// costs one memory round trip per input rather than one per value a thread holds.
-__global__ void __launch_bounds__(256)
-add_rms_norm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ delta,
-                    const float* __restrict__ planes, int splits, const uint16_t* __restrict__ w,
-                    uint16_t* __restrict__ res, uint16_t* __restrict__ y, int8_t* __restrict__ q,
-                    float* __restrict__ qs, uint8_t* __restrict__ q8, float* __restrict__ q8s, int rows, int n,
-                    float eps) {
+struct NormArgs {
+  const uint16_t *x, *delta;
+  const float* planes;
+  int splits;
+  const uint16_t* w;
+  uint16_t *res, *y;
+  int8_t* q;
+  float* qs;
+  uint8_t* q8;
+  float* q8s;
+  int rows, n;
+  float eps;
+};
+
+// What becomes of the normed row besides y.
+enum { kNormOnly, kNormInt8, kNormFp8 };
+
+// 1/sqrt(mean + eps) of a row whose squares' partial sums lie in part[0 .. waves - 1]: summed in
+// fp64 (each square of a bf16 value is exact there and so is the sum of a hidden row's worth, which
+// makes it independent of the order), mean rounded to fp32, + eps and 1/sqrt in fp32, as torch's
+// rsqrt(mean + eps).
+__device__ __forceinline__ float norm_scale(const double* part, int waves, int n, float eps) {
+  double total = part[0];
+  for (int w = 1; w < waves; ++w) total += part[w];
+  return 1.0f / sqrtf((float)(total / (double)n) + eps);
+}
+
+// One workgroup per row of n = 8 nc values, U chunks of 8 per thread, nc <= 1024 U: the row stays in
+// registers between its two passes and every load (x, delta or the planes, w) is issued before any
+// is used. delta: bf16 [rows][n] or (PLANES) fp32 planes [splits][rows][n], or neither (plain
+// RMSNorm, no residual written). Bound by latency, so also by the instructions that a launch fetches
+// from a cold cache: the first form, eight guarded chunks per thread of 256 with every option in
+// each, was 43 KB of code and took 3.9 us per call in a graph (8 rows of 2560) where this one, 2 to
+// 5 KB, takes 2.7.
+template <int U, bool PLANES, int QUANT>
+__global__ void __launch_bounds__(1024) norm_row_kernel(NormArgs a) {
+  extern __shared__ float rbuf[];  // kNormInt8: the normed row
+  __shared__ double part[16];
+  __shared__ float pmax[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
+  const int row = blockIdx.x, nc = a.n >> 3;
+  const size_t base = (size_t)row * a.n;
+  const bool add = PLANES || a.delta != nullptr;
+  uint4 xv[U], dv[U], wv[U];
+  u32x4 pv[U][2];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = tid + u * blockDim.x;
+    xv[u] = dv[u] = wv[u] = uint4{0u, 0u, 0u, 0u};
+    if (c < nc) {
+      xv[u] = ld16(a.x + base + 8 * c);
+      if (!PLANES && add) dv[u] = ld16(a.delta + base + 8 * c);
+      wv[u] = ld16(a.w + 8 * c);
+    }
+  }
+  float d[U][8];
+  if constexpr (PLANES) {  // slice-order fp32 sums
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) d[u][i] = 0.f;
+#pragma unroll 4
+    for (int sl = 0; sl < a.splits; ++sl) {
+      const float* pl = a.planes + (size_t)sl * a.rows * a.n + base;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int c = tid + u * blockDim.x;
+        if (c < nc) {
+          pv[u][0] = *gmem(reinterpret_cast<const u32x4*>(pl + 8 * c));
+          pv[u][1] = *gmem(reinterpret_cast<const u32x4*>(pl + 8 * c + 4));
+#pragma unroll
+          for (int i = 0; i < 8; ++i) d[u][i] += __uint_as_float(pv[u][i >> 2][i & 3]);
+        }
+      }
+    }
+  }
+  float r[U][8];
+  double ss = 0.0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = tid + u * blockDim.x;
+    const uint32_t xs[4] = {xv[u].x, xv[u].y, xv[u].z, xv[u].w};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[u][i] = bf2f((xs[i >> 1] >> (16 * (i & 1))) & 0xffffu);
+    if (add && c < nc) {
+      const uint32_t ds[4] = {dv[u].x, dv[u].y, dv[u].z, dv[u].w};
+      // bf16 rounding by the hardware's pair conversion (the integer rounding's bits for every
+      // value but a NaN, which then gets the integer rounding's form).
+      uint32_t rp[4], nan = 0u;
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        float d0 = bf2f(ds[i >> 1] & 0xffffu), d1 = bf2f(ds[i >> 1] >> 16);
+        if constexpr (PLANES) {
+          const uint32_t dp = bf16_pair_hw(d[u][i], d[u][i + 1]);
+          nan |= bf16_nan_bits(dp);
+          d0 = bf2f(dp & 0xffffu);
+          d1 = bf2f(dp >> 16);
+        }
+        rp[i >> 1] = bf16_pair_hw(r[u][i] + d0, r[u][i + 1] + d1);
+        nan |= bf16_nan_bits(rp[i >> 1]);
+      }
+      if (nan != 0u) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rp[i] = bf16_canonical_nan(rp[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) r[u][i] = bf2f((rp[i >> 1] >> (16 * (i & 1))) & 0xffffu);
+      if (a.res) *gmem(reinterpret_cast<u32x4*>(a.res + base + 8 * c)) = u32x4{rp[0], rp[1], rp[2], rp[3]};
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss += (double)r[u][i] * (double)r[u][i];
+  }
+  ss = wave_sum_last(ss);
+  if (lane == 63) part[wave] = ss;
+  __syncthreads();
+  const float scale = norm_scale(part, waves, a.n, a.eps);
+  uint32_t vp[U][4];
+  float mx = 0.f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int c = tid + u * blockDim.x;
+    const uint32_t ws[4] = {wv[u].x, wv[u].y, wv[u].z, wv[u].w};
+    uint32_t nan = 0u;
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {  // as above
+      const uint32_t t = bf16_pair_hw(r[u][i] * scale, r[u][i + 1] * scale);
+      vp[u][i >> 1] = bf16_pair_hw(bf2f(t & 0xffffu) * bf2f(ws[i >> 1] & 0xffffu),
+                                   bf2f(t >> 16) * bf2f(ws[i >> 1] >> 16));
+      nan |= bf16_nan_bits(t) | bf16_nan_bits(vp[u][i >> 1]);
+    }
+    if (nan != 0u) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) vp[u][i] = bf16_canonical_nan(vp[u][i]);
+    }
+    if (c < nc) {
+      if (a.y) *gmem(reinterpret_cast<u32x4*>(a.y + base + 8 * c)) = u32x4{vp[u][0], vp[u][1], vp[u][2], vp[u][3]};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float v = bf2f((vp[u][i >> 1] >> (16 * (i & 1))) & 0xffffu);
+        if constexpr (QUANT == kNormInt8) rbuf[8 * c + i] = v;
+        if constexpr (QUANT == kNormFp8) mx = fmaxf(mx, fabsf(v));
+      }
+    }
+  }
+  if constexpr (QUANT == kNormFp8) {
+    // per-token e4m3 quantize of the normed row: scale = max(amax / 448, 1e-12), codes e4m3(x / scale)
+    mx = wave_max_last(mx);
+    if (lane == 63) pmax[wave] = mx;
+    __syncthreads();
+    mx = pmax[0];
+    for (int w = 1; w < waves; ++w) mx = fmaxf(mx, pmax[w]);
+    const float sc = fmaxf(mx / 448.f, 1e-12f), yr = 1.f / sc;
+    if (tid == 0) a.q8s[row] = sc;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int c = tid + u * blockDim.x;
+      if (c < nc) {
+        const uint2 e = e4m3_chunk(uint4{vp[u][0], vp[u][1], vp[u][2], vp[u][3]}, sc, yr);
+        *gmem(reinterpret_cast<u32x2*>(a.q8 + base + 8 * c)) = u32x2{e.x, e.y};
+      }
+    }
+  }
+  if constexpr (QUANT == kNormInt8) {
+    // INT8 activation quantize per 64-group, fragment order (cuda_int8.py:30-44).
+    __syncthreads();
+    const int groups = a.n / 64;
+    for (int g = wave; g < groups; g += waves) {
+      const int nat = (lane >> 4) * 4 + ((lane & 15) >> 2) * 16 + (lane & 3);
+      const float v = rbuf[g * 64 + nat];
+      const float amax = wave_max(fabsf(v));
+      const float s = fmaxf(amax / 127.f, 1e-20f);
+      a.q[base + g * 64 + lane] = (int8_t)(int)rintf(v / s);
+      if (lane == 0) a.qs[(size_t)row * groups + g] = s;
+    }
+  }
+}
+
+// Rows of any length, a value at a time (n not a multiple of 8; no quantized output).
+__global__ void __launch_bounds__(256) norm_row_scalar_kernel(NormArgs a) {
   extern __shared__ float rbuf[];  // the row's residual, fp32
   __shared__ double part[4];
   const int row = blockIdx.x;
-  const size_t base = (size_t)row * n;
-  const bool add = delta != nullptr || planes != nullptr;
-  // Sum of squares in fp64: each square of a bf16 value is exact there and so is the sum of
-  // a hidden row's worth, which makes the scale independent of the summation order.
+  const size_t base = (size_t)row * a.n;
   double ss = 0.0;
-  const bool vec = (n & 7) == 0;
-  if (vec) {
-    const int nc = n >> 3;
-    uint4 xv[kNormChunks], dv[kNormChunks];
-#pragma unroll
-    for (int u = 0; u < kNormChunks; ++u) {
-      const int c = threadIdx.x + u * 256;
-      if (c < nc) {
-        xv[u] = ld16(x + base + 8 * c);
-        if (delta) dv[u] = ld16(delta + base + 8 * c);
-      }
-    }
-    float d[kNormChunks][8];
-    if (planes) {  // slice-order fp32 sums, each slice's loads of every chunk issued together
-#pragma unroll
-      for (int u = 0; u < kNormChunks; ++u)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) d[u][i] = 0.f;
-      for (int sl = 0; sl < splits; ++sl) {
-        const float* pl = planes + (size_t)sl * rows * n + base;
-        u32x4 pv[kNormChunks][2];
-#pragma unroll
-        for (int u = 0; u < kNormChunks; ++u) {
-          const int c = threadIdx.x + u * 256;
-          if (c < nc) {
-            pv[u][0] = *reinterpret_cast<const u32x4*>(pl + 8 * c);
-            pv[u][1] = *reinterpret_cast<const u32x4*>(pl + 8 * c + 4);
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < kNormChunks; ++u) {
-          const int c = threadIdx.x + u * 256;
-          if (c < nc)
-#pragma unroll
-            for (int i = 0; i < 8; ++i) d[u][i] += __uint_as_float(pv[u][i >> 2][i & 3]);
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kNormChunks; ++u) {
-      const int c = threadIdx.x + u * 256;
-      if (c >= nc) continue;
-      const uint32_t xs[4] = {xv[u].x, xv[u].y, xv[u].z, xv[u].w};
-      float r[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) r[i] = bf2f((xs[i >> 1] >> (16 * (i & 1))) & 0xffffu);
-      if (add) {
-        const uint32_t ds[4] = {dv[u].x, dv[u].y, dv[u].z, dv[u].w};
-        // bf16 rounding by the hardware's pair conversion (the integer rounding's bits for every
-        // value but a NaN); a chunk meeting a NaN is redone the integer way.
-        uint32_t rp[4], nan = 0u;
-#pragma unroll
-        for (int i = 0; i < 8; i += 2) {
-          float dd0, dd1;
-          if (planes) {
-            const uint32_t dp = bf16_pair_hw(d[u][i], d[u][i + 1]);
-            nan |= bf16_nan_bits(dp);
-            dd0 = bf2f(dp & 0xffffu);
-            dd1 = bf2f(dp >> 16);
-          } else {
-            dd0 = bf2f(ds[i >> 1] & 0xffffu);
-            dd1 = bf2f(ds[i >> 1] >> 16);
-          }
-          rp[i >> 1] = bf16_pair_hw(r[i] + dd0, r[i + 1] + dd1);
-          nan |= bf16_nan_bits(rp[i >> 1]);
-        }
-        if (nan == 0u) {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) r[i] = bf2f((rp[i >> 1] >> (16 * (i & 1))) & 0xffffu);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const float dd = planes ? round_bf(d[u][i]) : bf2f((ds[i >> 1] >> (16 * (i & 1))) & 0xffffu);
-            r[i] = round_bf(r[i] + dd);
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) rp[i] = pack_bf2(r[2 * i], r[2 * i + 1]);
-        }
-        if (res) *reinterpret_cast<u32x4*>(res + base + 8 * c) = u32x4{rp[0], rp[1], rp[2], rp[3]};
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        rbuf[8 * c + i] = r[i];
-        ss += (double)r[i] * (double)r[i];
-      }
-    }
-  } else {
-    for (int c = threadIdx.x; c < n; c += 256) {
-      float r = bf2f(x[base + c]);
-      if (add) {
-        float d;
-        if (planes) {
-          d = 0.f;
-          for (int sl = 0; sl < splits; ++sl) d += planes[(size_t)sl * rows * n + base + c];
-          d = round_bf(d);
-        } else {
-          d = bf2f(delta[base + c]);
-        }
-        r = round_bf(r + d);
-        if (res) res[base + c] = f2bf(r);
-      }
-      rbuf[c] = r;
-      ss += (double)r * (double)r;
-    }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
-  __syncthreads();
-  const double total = ((part[0] + part[1]) + part[2]) + part[3];
-  // mean rounded to fp32, + eps and 1/sqrt in fp32, as torch's rsqrt(mean + eps)
-  const float scale = 1.0f / sqrtf((float)(total / (double)n) + eps);
-  if (vec) {
-    const int nc = n >> 3;
-    uint4 wv[kNormChunks];
-#pragma unroll
-    for (int u = 0; u < kNormChunks; ++u) {
-      const int c = threadIdx.x + u * 256;
-      if (c < nc) wv[u] = ld16(w + 8 * c);
-    }
-#pragma unroll
-    for (int u = 0; u < kNormChunks; ++u) {
-      const int c = threadIdx.x + u * 256;
-      if (c >= nc) continue;
-      const uint32_t ws[4] = {wv[u].x, wv[u].y, wv[u].z, wv[u].w};
-      float v[8];
-      uint32_t vp[4], nan = 0u;
-#pragma unroll
-      for (int i = 0; i < 8; i += 2) {  // as above: the pair conversion, the integer way on a NaN
-        const uint32_t t = bf16_pair_hw(rbuf[8 * c + i] * scale, rbuf[8 * c + i + 1] * scale);
-        vp[i >> 1] = bf16_pair_hw(bf2f(t & 0xffffu) * bf2f(ws[i >> 1] & 0xffffu),
-                                  bf2f(t >> 16) * bf2f(ws[i >> 1] >> 16));
-        nan |= bf16_nan_bits(t) | bf16_nan_bits(vp[i >> 1]);
-      }
-      if (nan == 0u) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = bf2f((vp[i >> 1] >> (16 * (i & 1))) & 0xffffu);
+  for (int c = threadIdx.x; c < a.n; c += 256) {
+    float r = bf2f(a.x[base + c]);
+    if (a.delta != nullptr || a.planes != nullptr) {
+      float d;
+      if (a.planes) {
+        d = 0.f;
+        for (int sl = 0; sl < a.splits; ++sl) d += a.planes[(size_t)sl * a.rows * a.n + base + c];
+        d = round_bf(d);
       } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          v[i] = round_bf(round_bf(rbuf[8 * c + i] * scale) * bf2f((ws[i >> 1] >> (16 * (i & 1))) & 0xffffu));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) vp[i] = pack_bf2(v[2 * i], v[2 * i + 1]);
+        d = bf2f(a.delta[base + c]);
       }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) rbuf[8 * c + i] = v[i];
-      if (y) *reinterpret_cast<u32x4*>(y + base + 8 * c) = u32x4{vp[0], vp[1], vp[2], vp[3]};
+      r = round_bf(r + d);
+      if (a.res) a.res[base + c] = f2bf(r);
     }
-  } else {
-    for (int c = threadIdx.x; c < n; c += 256) {
-      const float v = round_bf(round_bf(rbuf[c] * scale) * bf2f(w[c]));
-      rbuf[c] = v;
-      if (y) y[base + c] = f2bf(v);
-    }
+    rbuf[c] = r;
+    ss += (double)r * (double)r;
   }
-  if (q8) {
-    // FP8 per-token activation quantize of the normed row (every value is a bf16 value, so its
-    // top 16 bits are its bf16 bits, a NaN's the integer rounding's sign | 0x7FC0 form):
-    // scale = max(amax / 448, 1e-12), codes e4m3(x / scale).
-    __shared__ float pmax[4];
-    __syncthreads();
-    float mx = 0.f;
-    for (int c = threadIdx.x; c < n; c += 256) mx = fmaxf(mx, fabsf(rbuf[c]));
-    mx = wave_max(mx);
-    if ((threadIdx.x & 63) == 0) pmax[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    const float sc = fmaxf(fmaxf(fmaxf(pmax[0], pmax[1]), fmaxf(pmax[2], pmax[3])) / 448.f, 1e-12f);
-    const float yr = 1.f / sc;
-    if (threadIdx.x == 0) q8s[row] = sc;
-    for (int c8 = threadIdx.x; c8 < (n >> 3); c8 += 256) {
-      uint32_t pk[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        pk[i] = (__float_as_uint(rbuf[8 * c8 + 2 * i]) >> 16) | (__float_as_uint(rbuf[8 * c8 + 2 * i + 1]) & 0xffff0000u);
-      *reinterpret_cast<uint2*>(q8 + base + 8 * c8) = e4m3_chunk(uint4{pk[0], pk[1], pk[2], pk[3]}, sc, yr);
-    }
-    return;
-  }
-  if (!q) return;
-  // INT8 activation quantize per 64-group, fragment order (cuda_int8.py:30-44).
+  ss = wave_sum_last(ss);
+  if ((threadIdx.x & 63) == 63) part[threadIdx.x >> 6] = ss;
   __syncthreads();
-  const int lane = threadIdx.x & 63;
-  const int groups = n / 64;
-  for (int g = threadIdx.x >> 6; g < groups; g += 4) {
-    const int nat = (lane >> 4) * 4 + ((lane & 15) >> 2) * 16 + (lane & 3);
-    const float v = rbuf[g * 64 + nat];
-    const float amax = wave_max(fabsf(v));
-    const float s = fmaxf(amax / 127.f, 1e-20f);
-    q[base + g * 64 + lane] = (int8_t)(int)rintf(v / s);
-    if (lane == 0) qs[(size_t)row * groups + g] = s;
-  }
+  const float scale = norm_scale(part, 4, a.n, a.eps);
+  for (int c = threadIdx.x; c < a.n; c += 256)
+    if (a.y) a.y[base + c] = f2bf(round_bf(rbuf[c] * scale) * bf2f(a.w[c]));
+}
+
+template <int U, int QUANT>
+void launch_norm_row(const NormArgs& a, hipStream_t st) {
+  const int nc = a.n >> 3, threads = ((nc + U - 1) / U + 63) / 64 * 64;
+  const size_t lds = QUANT == kNormInt8 ? a.n * sizeof(float) : 0;
+  if (a.planes) norm_row_kernel<U, true, QUANT><<<a.rows, threads, lds, st>>>(a);
+  else norm_row_kernel<U, false, QUANT><<<a.rows, threads, lds, st>>>(a);
+}
+
+// Threads for every chunk of a row up to 8192 values, two chunks per thread above (n <= 16384).
+template <int QUANT>
+void launch_norm(const NormArgs& a, hipStream_t st) {
+  if (a.n % 8) norm_row_scalar_kernel<<<a.rows, 256, a.n * sizeof(float), st>>>(a);
+  else if (a.n <= 8192) launch_norm_row<1, QUANT>(a, st);
+  else launch_norm_row<2, QUANT>(a, st);
 }
 
 // gate_up: bf16 [rows][2I] or (planes != null) fp32 planes [splits][rows][2I].
@@ -310,9 +323,9 @@ int qlx_add_rms_norm(const void* x, const void* delta, const float* planes, int 
                      void* res, void* y, int rows, int n, float eps, void* stream) {
   QLX_REQUIRE(rows > 0 && n > 0 && n <= 16384, "rows=%d n=%d: rows must be > 0 and n in 1..16384", rows, n);
   QLX_REQUIRE(planes == nullptr || splits >= 1, "planes need splits >= 1");
-  add_rms_norm_kernel<<<rows, 256, n * sizeof(float), (hipStream_t)stream>>>(
-      (const uint16_t*)x, (const uint16_t*)delta, planes, splits, (const uint16_t*)w, (uint16_t*)res,
-      (uint16_t*)y, nullptr, nullptr, nullptr, nullptr, rows, n, eps);
+  launch_norm<kNormOnly>(NormArgs{(const uint16_t*)x, (const uint16_t*)delta, planes, splits, (const uint16_t*)w, (uint16_t*)res,
+                        (uint16_t*)y, nullptr, nullptr, nullptr, nullptr, rows, n, eps},
+                  (hipStream_t)stream);
   QLX_LAUNCH_CHECK("add_rms_norm");
 }
 
@@ -321,9 +334,9 @@ int qlx_add_norm_quant_int8(const void* x, const void* delta, const float* plane
                             void* stream) {
   QLX_REQUIRE(rows > 0 && n > 0 && n <= 16384 && n % 64 == 0, "n=%d must be a multiple of 64 up to 16384", n);
   QLX_REQUIRE(planes == nullptr || splits >= 1, "planes need splits >= 1");
-  add_rms_norm_kernel<<<rows, 256, n * sizeof(float), (hipStream_t)stream>>>(
-      (const uint16_t*)x, (const uint16_t*)delta, planes, splits, (const uint16_t*)w, (uint16_t*)res,
-      nullptr, (int8_t*)q, q_scale, nullptr, nullptr, rows, n, eps);
+  launch_norm<kNormInt8>(NormArgs{(const uint16_t*)x, (const uint16_t*)delta, planes, splits, (const uint16_t*)w, (uint16_t*)res,
+                        nullptr, (int8_t*)q, q_scale, nullptr, nullptr, rows, n, eps},
+                  (hipStream_t)stream);
   QLX_LAUNCH_CHECK("add_norm_quant_int8");
 }
 
@@ -332,9 +345,9 @@ int qlx_add_norm_quant_fp8(const void* x, const void* delta, const float* planes
   QLX_REQUIRE(rows > 0 && n > 0 && n <= 16384 && n % 8 == 0, "n=%d must be a multiple of 8 up to 16384", n);
   QLX_REQUIRE(planes == nullptr || splits >= 1, "planes need splits >= 1");
   QLX_REQUIRE(code != nullptr && scale != nullptr, "codes and scales are required");
-  add_rms_norm_kernel<<<rows, 256, n * sizeof(float), (hipStream_t)stream>>>(
-      (const uint16_t*)x, (const uint16_t*)delta, planes, splits, (const uint16_t*)w, (uint16_t*)res,
-      (uint16_t*)y, nullptr, nullptr, (uint8_t*)code, scale, rows, n, eps);
+  launch_norm<kNormFp8>(NormArgs{(const uint16_t*)x, (const uint16_t*)delta, planes, splits, (const uint16_t*)w, (uint16_t*)res,
+                        (uint16_t*)y, nullptr, nullptr, (uint8_t*)code, scale, rows, n, eps},
+                  (hipStream_t)stream);
   QLX_LAUNCH_CHECK("add_norm_quant_fp8");
 }
 

@@ -327,33 +327,48 @@ row_major_ref_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
 
 // ---- FP8 e4m3 (fp8.py:20-28) ------------------------------------------------------------------
 
-// Per-token activation quantize: one block of 256 threads per row.
-__global__ void __launch_bounds__(256)
+// Per-token activation quantize: a block per row, U chunks of 8 values per thread, held in registers
+// between the maximum and the codes (U = 0: a loop that reads the row twice, for rows of over 16384).
+template <int U>
+__global__ void __launch_bounds__(1024)
 quantize_fp8_act_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ code,
                         float* __restrict__ scale, int k) {
-  __shared__ float part[4];
-  const int row = blockIdx.x;
-  const uint16_t* src = x + (size_t)row * k;
+  __shared__ float part[16];
+  const int row = blockIdx.x, lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+  const size_t base = (size_t)row * k;
   const int octets = k >> 3;
+  uint4 v[U ? U : 1];
   float amax = 0.f;
-  for (int o = threadIdx.x; o < octets; o += 256) {
-    const uint4 v = *reinterpret_cast<const uint4*>(src + 8 * o);
-    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+  if constexpr (U > 0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      amax = fmaxf(amax, fabsf(bf2f(d[j] & 0xffffu)));
-      amax = fmaxf(amax, fabsf(bf2f(d[j] >> 16)));
+    for (int u = 0; u < U; ++u) {
+      const int o = threadIdx.x + u * blockDim.x;
+      v[u] = uint4{0u, 0u, 0u, 0u};
+      if (o < octets) v[u] = *reinterpret_cast<const uint4*>(x + base + 8 * o);
     }
+#pragma unroll
+    for (int u = 0; u < U; ++u) amax = octet_amax(v[u], amax);
+  } else {
+    for (int o = threadIdx.x; o < octets; o += blockDim.x)
+      amax = octet_amax(*reinterpret_cast<const uint4*>(x + base + 8 * o), amax);
   }
-  amax = wave_max(amax);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = amax;
+  amax = wave_max_last(amax);
+  if (lane == 63) part[threadIdx.x >> 6] = amax;
   __syncthreads();
-  amax = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+  amax = part[0];
+  for (int w = 1; w < waves; ++w) amax = fmaxf(amax, part[w]);
   const float s = fmaxf(amax / 448.f, 1e-12f), y = 1.f / s;
   if (threadIdx.x == 0) scale[row] = s;
-  for (int o = threadIdx.x; o < octets; o += 256)
-    *reinterpret_cast<uint2*>(code + (size_t)row * k + 8 * o) =
-        e4m3_chunk(*reinterpret_cast<const uint4*>(src + 8 * o), s, y);
+  if constexpr (U > 0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int o = threadIdx.x + u * blockDim.x;
+      if (o < octets) *reinterpret_cast<uint2*>(code + base + 8 * o) = e4m3_chunk(v[u], s, y);
+    }
+  } else {
+    for (int o = threadIdx.x; o < octets; o += blockDim.x)
+      *reinterpret_cast<uint2*>(code + base + 8 * o) = e4m3_chunk(*reinterpret_cast<const uint4*>(x + base + 8 * o), s, y);
+  }
 }
 
 // Every input the FP8 quantizers can see, through e4m3_chunk and through e4m3_of_quotient: a
@@ -504,8 +519,12 @@ int qlx_quantize_fp8_weight(const void* w, void* code, void* scale, int rows, in
 
 int qlx_quantize_fp8_act(const void* x, void* code, float* scale, int m, int k, void* stream) {
   QLX_REQUIRE(m > 0 && k > 0 && k % 8 == 0, "activation K=%d must be a positive multiple of 8", k);
-  quantize_fp8_act_kernel<<<m, 256, 0, (hipStream_t)stream>>>((const uint16_t*)x, (uint8_t*)code,
-                                                              scale, k);
+  // Threads for every 8 values of a row up to 8192, two pieces per thread to 16384: 256 threads that
+  // read a row twice took 2.80 and 4.20 us per call in a graph (8 rows of 2560, 9728), these 2.38 and 2.85.
+  const int octets = k >> 3, u = octets <= 1024 ? 1 : (octets <= 2048 ? 2 : 0);
+  const int threads = u ? ((octets + u - 1) / u + 63) / 64 * 64 : 1024;
+  const auto fn = u == 1 ? quantize_fp8_act_kernel<1> : (u == 2 ? quantize_fp8_act_kernel<2> : quantize_fp8_act_kernel<0>);
+  fn<<<m, threads, 0, (hipStream_t)stream>>>((const uint16_t*)x, (uint8_t*)code, scale, k);
   QLX_LAUNCH_CHECK("quantize_fp8_act");
 }
 

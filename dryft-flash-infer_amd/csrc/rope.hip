@@ -2,9 +2,9 @@
 // (engine/kernels/rope.py:24-60 `_norm_rope`, :63-92 q/kv kernels, :125-166 the fused Q/K/V
 // kernel, :169-218 the split-K planes variant, :96-122 the INT8 cache writes).
 //
-// Eight lanes per 128-value head (rope_common.h: the lane layout and the roundings, those of
-// engine/kernels/reference.py:31-46). A workgroup of 256 threads covers 32 heads of one row:
-// Q heads, then K heads (whose lanes also move the V head).
+// Sixteen lanes per 128-value head (rope_common.h: the lane layout and the roundings, those of
+// engine/kernels/reference.py:31-46). A workgroup of 256 threads covers 16 heads of one row: Q heads,
+// then K heads, then V heads.
 // From planes, x = bf16(sum of the fp32 planes in slice order) (rope.py:169-176).
 // INT8 cache: per (token, head) scale max(amax |y|, 1e-12) / 127, codes
 // clamp(floor(y / scale + 0.5), -127, 127) (rope.py:108-118).
@@ -15,150 +15,152 @@ namespace qlx {
 
 struct RopeArgs {
   qlx_rope_args p;
-  int heads;  // n_q + n_kv
+  int heads;  // n_q + 2 n_kv
 };
 
-// 8 values of row `row` at column `col`: bf16 from qkv, or bf16(sum of the planes).
-__device__ __forceinline__ void load8(const qlx_rope_args& p, int row, long long col, float* f) {
-  if (p.planes == nullptr) {
-    const uint16_t* x = reinterpret_cast<const uint16_t*>(p.qkv) + (size_t)row * p.stride + col;
-    unpack8(*gmem(reinterpret_cast<const u32x4*>(x)), f);
-    return;
+// 4 values of row `row` at column `col`, as bf16 pairs: read from qkv, or the planes' slice-order
+// sums rounded once.
+template <bool PLANES>
+__device__ __forceinline__ u32x2 load4(const qlx_rope_args& p, int row, long long col) {
+  if constexpr (!PLANES) {
+    return *gmem(reinterpret_cast<const u32x2*>(reinterpret_cast<const uint16_t*>(p.qkv) + (size_t)row * p.stride + col));
+  } else {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < p.splits; ++s) {
+      const f32x4 v = *gmem(reinterpret_cast<const f32x4*>(p.planes + ((size_t)s * p.rows + row) * p.stride + col));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] += v[i];
+    }
+    return u32x2{bf16_canonical_nan(bf16_pair_hw(acc[0], acc[1])), bf16_canonical_nan(bf16_pair_hw(acc[2], acc[3]))};
   }
-  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < p.splits; ++s) {
-    const float* pp = p.planes + ((size_t)s * p.rows + row) * p.stride + col;
-    const f32x4 lo = *gmem(reinterpret_cast<const f32x4*>(pp));
-    const f32x4 hi = *gmem(reinterpret_cast<const f32x4*>(pp + 4));
+}
+
+__device__ __forceinline__ void unpack4(u32x2 d, float* f) {
+  f[0] = bf2f(d[0] & 0xffffu), f[1] = bf2f(d[0] >> 16), f[2] = bf2f(d[1] & 0xffffu), f[3] = bf2f(d[1] >> 16);
+}
+
+// clamp(floor(f / sc + 0.5), -127, 127) of 4 values. y = 1 / sc: the quotient is the IEEE one wherever
+// it can reach a code other than 0 (quotient_by_reciprocal); over an infinite scale finite values
+// give 0, the others a NaN, which the clamp turns into -127.
+__device__ __forceinline__ void store_int8(int8_t* dst, const float* f, float sc, float y) {
+  uint32_t d = 0u;
+  if (sc <= 3.40282347e38f) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      acc[i] += lo[i];
-      acc[4 + i] += hi[i];
+      const float c = fminf(fmaxf(floorf(quotient_by_reciprocal(f[i], sc, y) + 0.5f), -127.f), 127.f);
+      d |= ((uint32_t)(int)c & 0xffu) << (8 * i);
     }
-  }
+  } else {
 #pragma unroll
-  for (int i = 0; i < 8; ++i) f[i] = round_bf(acc[i]);
+    for (int i = 0; i < 4; ++i) d |= (fabsf(f[i]) <= 3.40282347e38f ? 0u : 0x81u) << (8 * i);
+  }
+  *gmem(reinterpret_cast<uint32_t*>(dst)) = d;
 }
 
-__device__ __forceinline__ void store_int8(int8_t* dst, const float* f, float sc) {
-  uint32_t d[2] = {0u, 0u};
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float c = fminf(fmaxf(floorf(f[i] / sc + 0.5f), -127.f), 127.f);
-    d[i >> 2] |= ((uint32_t)(int)c & 0xffu) << (8 * (i & 3));
-  }
-  *gmem(reinterpret_cast<u32x2*>(dst)) = u32x2{d[0], d[1]};
-}
-
-// Max over the 8 lanes of a head (lanes 8 h .. 8 h + 7 of the wave).
+// Max over the 16 lanes of a head.
 __device__ __forceinline__ float head_max(float v) {
   v = fmaxf(v, __shfl_xor(v, 1, 64));
   v = fmaxf(v, __shfl_xor(v, 2, 64));
-  return fmaxf(v, __shfl_xor(v, 4, 64));
+  v = fmaxf(v, __shfl_xor(v, 4, 64));
+  return fmaxf(v, __shfl_xor(v, 8, 64));
 }
 
+// A lane's two groups of 4 values (bf16 pairs lo, hi: dims 4 j .., 64 + 4 j ..) into head slot `slot`
+// of a bf16 cache, or quantized into an INT8 one with its scale.
+template <bool INT8>
+__device__ __forceinline__ void write_head(void* cache, float* scales, size_t slot, int j, const u32x2& lo, const u32x2& hi,
+                                           bool writes) {
+  if constexpr (INT8) {
+    float fl[4], fh[4];
+    unpack4(lo, fl);
+    unpack4(hi, fh);
+    float amax = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) amax = fmaxf(amax, fmaxf(fabsf(fl[i]), fabsf(fh[i])));
+    const float sc = fmaxf(head_max(amax), 1e-12f) / 127.0f, y = 1.0f / sc;
+    if (!writes) return;
+    int8_t* dst = reinterpret_cast<int8_t*>(cache) + slot * 128;
+    store_int8(dst + 4 * j, fl, sc, y);
+    store_int8(dst + 64 + 4 * j, fh, sc, y);
+    if (j == 0) scales[slot] = sc;
+  } else {
+    if (!writes) return;
+    uint16_t* dst = reinterpret_cast<uint16_t*>(cache) + slot * 128;
+    *gmem(reinterpret_cast<u32x2*>(dst + 4 * j)) = lo;
+    *gmem(reinterpret_cast<u32x2*>(dst + 64 + 4 * j)) = hi;
+  }
+}
+
+// A launch is a chain of two memory round trips and a wave's instructions, fetched cold: one
+// instance per source and cache type, 16 lanes per head (half the values, so half the instructions, of
+// 8), value heads on lanes of their own. us per call in a graph at 1 / 64 rows of 32 + 8 heads: bf16
+// cache 3.56 / 3.78 -> 2.45 / 2.85, INT8 4.49 / 4.76 -> 2.90 / 3.29 (8 lanes per head, all options in
+// one kernel of 19 KB, a value head read by its key's lanes).
+template <bool PLANES, bool INT8>
 __global__ void __launch_bounds__(256) rope_kernel(RopeArgs ra) {
   const qlx_rope_args& p = ra.p;
   const int row = blockIdx.x;
-  const int hh = blockIdx.y * 32 + (threadIdx.x >> 3);
-  const int j = threadIdx.x & 7;
-  // Lanes past the last head compute on head 0's data and store nothing (a head's 8 lanes
+  const int hh = blockIdx.y * 16 + (threadIdx.x >> 4);
+  const int j = threadIdx.x & 15;
+  // Lanes past the last head compute on head 0's data and store nothing (a head's 16 lanes
   // take the same branch, and no lane leaves before the shuffles).
   const bool active = hh < ra.heads;
   const int h = active ? hh : 0;
-  const bool is_q = h < p.n_q;
-  const int kvh = h - p.n_q;
-  const long long col = is_q ? p.q_col + (long long)h * 128 : p.k_col + (long long)kvh * 128;
+  const bool is_q = h < p.n_q, is_v = h >= p.n_q + p.n_kv;
+  const int kvh = is_v ? h - p.n_q - p.n_kv : h - p.n_q;
+  const long long col = is_q ? p.q_col + (long long)h * 128 : (is_v ? p.v_col : p.k_col) + (long long)kvh * 128;
 
   // The position first: the cos/sin rows it selects are the second of two dependent loads.
   const int tok = row % p.seq_len;
   const long long pos = p.pos_int64 ? reinterpret_cast<const long long*>(p.positions)[tok]
                                     : (long long)reinterpret_cast<const int*>(p.positions)[tok];
+  u32x2 lo = load4<PLANES>(p, row, col + 4 * j), hi = load4<PLANES>(p, row, col + 64 + 4 * j);
   const bool in_table = pos >= 0 && pos < p.table_rows;
-  const long long tp = in_table ? pos : 0;
-  float cl[8], ch[8], sl[8], sh[8];
-  const uint16_t* cs = reinterpret_cast<const uint16_t*>(p.cos) + (size_t)tp * 128;
-  const uint16_t* sn = reinterpret_cast<const uint16_t*>(p.sin) + (size_t)tp * 128;
-  unpack8(*gmem(reinterpret_cast<const u32x4*>(cs + 8 * j)), cl);
-  unpack8(*gmem(reinterpret_cast<const u32x4*>(cs + 64 + 8 * j)), ch);
-  unpack8(*gmem(reinterpret_cast<const u32x4*>(sn + 8 * j)), sl);
-  unpack8(*gmem(reinterpret_cast<const u32x4*>(sn + 64 + 8 * j)), sh);
-
-  float xl[8], xh[8];
-  load8(p, row, col + 8 * j, xl);
-  load8(p, row, col + 64 + 8 * j, xh);
-  const uint16_t* gain = reinterpret_cast<const uint16_t*>(is_q ? p.q_norm_w : p.k_norm_w);
-  float wl[8], wh[8];
-  unpack8(*gmem(reinterpret_cast<const u32x4*>(gain + 8 * j)), wl);
-  unpack8(*gmem(reinterpret_cast<const u32x4*>(gain + 64 + 8 * j)), wh);
-  float yl[8], yh[8];
-  uint32_t ylp[4], yhp[4];
-  rope_norm_rotate(xl, xh, wl, wh, cl, ch, sl, sh, p.eps, yl, yh, ylp, yhp);
-
-  if (is_q) {
-    if (!active) return;
-    uint16_t* q = reinterpret_cast<uint16_t*>(p.q_out) + (size_t)row * p.n_q * 128 + (size_t)h * 128;
-    if (!in_table) {  // a position outside the cos/sin table: the head reads as NaN
-#pragma unroll
-      for (int i = 0; i < 8; ++i) yl[i] = yh[i] = __builtin_nanf("");
-    }
-    if (!in_table) {
-      *gmem(reinterpret_cast<u32x4*>(q + 8 * j)) = pack8(yl);
-      *gmem(reinterpret_cast<u32x4*>(q + 64 + 8 * j)) = pack8(yh);
-    } else {
-      *gmem(reinterpret_cast<u32x4*>(q + 8 * j)) = u32x4{ylp[0], ylp[1], ylp[2], ylp[3]};
-      *gmem(reinterpret_cast<u32x4*>(q + 64 + 8 * j)) = u32x4{yhp[0], yhp[1], yhp[2], yhp[3]};
-    }
-    return;
-  }
-
-  // K head kvh: rotated K and the raw V head to slot pos of sequence row / seq_len.
-  float vl[8], vh[8];
-  const long long vcol = p.v_col + (long long)kvh * 128;
-  load8(p, row, vcol + 8 * j, vl);
-  load8(p, row, vcol + 64 + 8 * j, vh);
-  const bool writes = active && in_table && pos < p.capacity;
   const int seq = row / p.seq_len;
+  const bool writes = active && in_table && pos < p.capacity;
+
+  if (!is_v) {
+    const uint16_t* gain = reinterpret_cast<const uint16_t*>(is_q ? p.q_norm_w : p.k_norm_w);
+    const u32x2 wlr = *gmem(reinterpret_cast<const u32x2*>(gain + 4 * j)),
+                whr = *gmem(reinterpret_cast<const u32x2*>(gain + 64 + 4 * j));
+    const long long tp = in_table ? pos : 0;
+    const uint16_t* cs = reinterpret_cast<const uint16_t*>(p.cos) + (size_t)tp * 128 + 4 * j;
+    const uint16_t* sn = reinterpret_cast<const uint16_t*>(p.sin) + (size_t)tp * 128 + 4 * j;
+    float cl[4], ch[4], sl[4], sh[4], xl[4], xh[4], wl[4], wh[4], yl[4], yh[4];
+    unpack4(*gmem(reinterpret_cast<const u32x2*>(cs)), cl);
+    unpack4(*gmem(reinterpret_cast<const u32x2*>(cs + 64)), ch);
+    unpack4(*gmem(reinterpret_cast<const u32x2*>(sn)), sl);
+    unpack4(*gmem(reinterpret_cast<const u32x2*>(sn + 64)), sh);
+    unpack4(lo, xl);
+    unpack4(hi, xh);
+    unpack4(wlr, wl);
+    unpack4(whr, wh);
+    uint32_t ylp[2], yhp[2];
+    rope_norm_rotate<4>(xl, xh, wl, wh, cl, ch, sl, sh, p.eps, yl, yh, ylp, yhp);
+    lo = u32x2{ylp[0], ylp[1]}, hi = u32x2{yhp[0], yhp[1]};
+    if (is_q) {
+      if (!active) return;
+      // a position outside the cos/sin table: the head reads as NaN
+      if (!in_table) lo = hi = u32x2{0x7fc07fc0u, 0x7fc07fc0u};
+      uint16_t* q = reinterpret_cast<uint16_t*>(p.q_out) + (size_t)row * p.n_q * 128 + (size_t)h * 128 + 4 * j;
+      *gmem(reinterpret_cast<u32x2*>(q)) = lo;
+      *gmem(reinterpret_cast<u32x2*>(q + 64)) = hi;
+      return;
+    }
+  } else {
+    lo = u32x2{bf16_canonical_nan(lo[0]), bf16_canonical_nan(lo[1])};
+    hi = u32x2{bf16_canonical_nan(hi[0]), bf16_canonical_nan(hi[1])};
+  }
+
+  // The rotated K or the raw V head to slot pos of sequence row / seq_len.
   const size_t hs = (size_t)seq * p.n_kv + kvh;
-  const size_t slot = (hs * p.capacity + (size_t)(writes ? pos : 0)) * 128;
   if (p.k_copy != nullptr && active) {
-    const size_t cslot = (hs * p.seq_len + tok) * 128;
-    uint16_t* kc = reinterpret_cast<uint16_t*>(p.k_copy) + cslot;
-    uint16_t* vc = reinterpret_cast<uint16_t*>(p.v_copy) + cslot;
-    *gmem(reinterpret_cast<u32x4*>(kc + 8 * j)) = u32x4{ylp[0], ylp[1], ylp[2], ylp[3]};
-    *gmem(reinterpret_cast<u32x4*>(kc + 64 + 8 * j)) = u32x4{yhp[0], yhp[1], yhp[2], yhp[3]};
-    *gmem(reinterpret_cast<u32x4*>(vc + 8 * j)) = pack8(vl);
-    *gmem(reinterpret_cast<u32x4*>(vc + 64 + 8 * j)) = pack8(vh);
+    uint16_t* copy = reinterpret_cast<uint16_t*>(is_v ? p.v_copy : p.k_copy) + (hs * p.seq_len + tok) * 128 + 4 * j;
+    *gmem(reinterpret_cast<u32x2*>(copy)) = lo;
+    *gmem(reinterpret_cast<u32x2*>(copy + 64)) = hi;
   }
-  if (p.k_scale != nullptr) {
-    float ka = 0.f, va = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      ka = fmaxf(ka, fmaxf(fabsf(yl[i]), fabsf(yh[i])));
-      va = fmaxf(va, fmaxf(fabsf(vl[i]), fabsf(vh[i])));
-    }
-    const float ks = fmaxf(head_max(ka), 1e-12f) / 127.0f;
-    const float vs = fmaxf(head_max(va), 1e-12f) / 127.0f;
-    if (!writes) return;
-    int8_t* kc = reinterpret_cast<int8_t*>(p.k_cache) + slot;
-    int8_t* vc = reinterpret_cast<int8_t*>(p.v_cache) + slot;
-    store_int8(kc + 8 * j, yl, ks);
-    store_int8(kc + 64 + 8 * j, yh, ks);
-    store_int8(vc + 8 * j, vl, vs);
-    store_int8(vc + 64 + 8 * j, vh, vs);
-    if (j == 0) {
-      p.k_scale[slot >> 7] = ks;
-      p.v_scale[slot >> 7] = vs;
-    }
-    return;
-  }
-  if (!writes) return;
-  uint16_t* kc = reinterpret_cast<uint16_t*>(p.k_cache) + slot;
-  uint16_t* vc = reinterpret_cast<uint16_t*>(p.v_cache) + slot;
-  *gmem(reinterpret_cast<u32x4*>(kc + 8 * j)) = u32x4{ylp[0], ylp[1], ylp[2], ylp[3]};
-  *gmem(reinterpret_cast<u32x4*>(kc + 64 + 8 * j)) = u32x4{yhp[0], yhp[1], yhp[2], yhp[3]};
-  *gmem(reinterpret_cast<u32x4*>(vc + 8 * j)) = pack8(vl);
-  *gmem(reinterpret_cast<u32x4*>(vc + 64 + 8 * j)) = pack8(vh);
+  write_head<INT8>(is_v ? p.v_cache : p.k_cache, is_v ? p.v_scale : p.k_scale,
+                   hs * p.capacity + (size_t)(writes ? pos : 0), j, lo, hi, writes);
 }
 
 }  // namespace qlx
@@ -186,8 +188,10 @@ extern "C" int qlx_qkv_norm_rope(const qlx_rope_args* args, void* stream) {
   QLX_REQUIRE((p.k_scale == nullptr) == (p.v_scale == nullptr), "norm_rope: give both cache scales or neither");
   QLX_REQUIRE((p.k_copy == nullptr) == (p.v_copy == nullptr), "norm_rope: give both bf16 copies or neither");
   if (p.rows == 0) return QLX_OK;
-  RopeArgs ra{p, p.n_q + p.n_kv};
-  const dim3 grid(p.rows, (ra.heads + 31) / 32);
-  rope_kernel<<<grid, 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(ra);
+  RopeArgs ra{p, p.n_q + 2 * p.n_kv};
+  const dim3 grid(p.rows, (ra.heads + 15) / 16);
+  const auto fn = p.planes ? (p.k_scale ? rope_kernel<true, true> : rope_kernel<true, false>)
+                           : (p.k_scale ? rope_kernel<false, true> : rope_kernel<false, false>);
+  fn<<<grid, 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(ra);
   QLX_LAUNCH_CHECK("norm_rope");
 }

@@ -31,21 +31,24 @@ __device__ __forceinline__ u32x4 pack8(const float* f) {
   return u32x4{d[0], d[1], d[2], d[3]};
 }
 
-// The lane's 16 values of a head (xl: dims 8 j + 0..7, xh: 64 + 8 j + 0..7), its norm gains
+// The lane's 2 N values of a head (N = 8 on 8 lanes: xl dims 8 j + 0..7, xh 64 + 8 j + 0..7; N = 4 on
+// 16 lanes likewise), its norm gains
 // (wl, wh), cos and sin (cl/ch, sl/sh) -> the rotated values, as floats (yl, yh) and bf16 pairs
-// (ylp, yhp). Every lane of the wave takes part (the head's lanes are 8 consecutive lanes whose
-// index differs in bits 0..2). Every rounding is to bf16, by the hardware's pair conversion
-// (the integer rounding's bits for every value but a NaN, checked on all 2^32 inputs); a lane
-// meeting a NaN redoes its values with the integer rounding.
+// (ylp, yhp). Every lane of the wave takes part (the head's lanes are consecutive lanes whose
+// index differs in the lowest bits). Every rounding is to bf16, by the hardware's pair conversion
+// (the integer rounding's bits for every value but a NaN, checked on all 2^32 inputs); results that
+// are NaNs get the integer rounding's form.
+template <int N = 8>
 __device__ __forceinline__ void rope_norm_rotate(const float* xl, const float* xh, const float* wl, const float* wh,
                                                  const float* cl, const float* ch, const float* sl, const float* sh,
                                                  float eps, float* yl, float* yh, uint32_t* ylp, uint32_t* yhp) {
   double ss = 0.0;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) ss += (double)xl[i] * (double)xl[i] + (double)xh[i] * (double)xh[i];
+  for (int i = 0; i < N; ++i) ss += (double)xl[i] * (double)xl[i] + (double)xh[i] * (double)xh[i];
   ss += __shfl_xor(ss, 1, 64);
   ss += __shfl_xor(ss, 2, 64);
   ss += __shfl_xor(ss, 4, 64);
+  if constexpr (N == 4) ss += __shfl_xor(ss, 8, 64);
   const float scale = 1.0f / sqrtf((float)(ss / 128.0) + eps);
   uint32_t nan = 0u;
   auto lo = [](uint32_t p) { return bf2f(p & 0xffffu); };
@@ -56,7 +59,7 @@ __device__ __forceinline__ void rope_norm_rotate(const float* xl, const float* x
     return p;
   };
 #pragma unroll
-  for (int i = 0; i < 8; i += 2) {
+  for (int i = 0; i < N; i += 2) {
     const uint32_t ta = pr(xl[i] * scale, xl[i + 1] * scale), tb = pr(xh[i] * scale, xh[i + 1] * scale);
     const uint32_t a = pr(lo(ta) * wl[i], hi(ta) * wl[i + 1]);  // n[8 j + i], n[8 j + i + 1]
     const uint32_t b = pr(lo(tb) * wh[i], hi(tb) * wh[i + 1]);  // n[64 + 8 j + i], ...
@@ -65,26 +68,17 @@ __device__ __forceinline__ void rope_norm_rotate(const float* xl, const float* x
     ylp[i >> 1] = pr(lo(p1) + lo(p2), hi(p1) + hi(p2));
     yhp[i >> 1] = pr(lo(p3) + lo(p4), hi(p3) + hi(p4));
   }
-  if (nan == 0u) {
+  if (nan != 0u) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      yl[i] = bf2f((ylp[i >> 1] >> (16 * (i & 1))) & 0xffffu);
-      yh[i] = bf2f((yhp[i >> 1] >> (16 * (i & 1))) & 0xffffu);
+    for (int i = 0; i < N / 2; ++i) {
+      ylp[i] = bf16_canonical_nan(ylp[i]);
+      yhp[i] = bf16_canonical_nan(yhp[i]);
     }
-  } else {
+  }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float a = round_bf(round_bf(xl[i] * scale) * wl[i]);  // n[8 j + i]
-      const float b = round_bf(round_bf(xh[i] * scale) * wh[i]);  // n[64 + 8 j + i]
-      yl[i] = round_bf(round_bf(a * cl[i]) + round_bf(-b * sl[i]));
-      yh[i] = round_bf(round_bf(b * ch[i]) + round_bf(a * sh[i]));
-    }
-    const u32x4 l = pack8(yl), h = pack8(yh);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      ylp[i] = l[i];
-      yhp[i] = h[i];
-    }
+  for (int i = 0; i < N; ++i) {
+    yl[i] = bf2f((ylp[i >> 1] >> (16 * (i & 1))) & 0xffffu);
+    yh[i] = bf2f((yhp[i >> 1] >> (16 * (i & 1))) & 0xffffu);
   }
 }
 
