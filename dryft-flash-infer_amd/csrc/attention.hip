@@ -48,11 +48,16 @@ struct AttnArgs {
   int cap, splits, T, G, H, R, heads;
 };
 
-// RT tiles of 16 query rows (R <= 16 RT). 256 threads; dynamic LDS 4 x R x 128 fp32.
+constexpr int W = 4;  // waves of a workgroup (8 measured the same or slower: INT8 13.8 against 12.7 us)
+
+// Splits in use: at least one block per wave each.
+__device__ __forceinline__ int live_splits(int nblk, int splits) { return max(1, min(splits, (nblk + W - 1) / W)); }
+
+// RT tiles of 16 query rows (R <= 16 RT); dynamic LDS W x R x 128 fp32.
 template <int RT, bool Q8>
-__global__ void __launch_bounds__(256) attn_kernel(AttnArgs a) {
-  extern __shared__ float wacc[];  // [4 waves][R][128]
-  __shared__ float wm[4][64], wl[4][64];
+__global__ void __launch_bounds__(64 * W) attn_kernel(AttnArgs a) {
+  extern __shared__ float wacc[];  // [W waves][R][128]
+  __shared__ float wm[W][64], wl[W][64];
   const int head = blockIdx.x, part = blockIdx.y;
   // wave index and position in scalar registers: block bounds and loop trips are wave-uniform
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -61,7 +66,7 @@ __global__ void __launch_bounds__(256) attn_kernel(AttnArgs a) {
   const int NQ = a.H * a.G;
   const size_t hb = (size_t)head * a.cap * 128;
   // Key blocks of 32 are dealt round-robin: block j to split j % S, and within the split to
-  // wave (j / S) % 4. A wave's first block is then known before the position is: its K/V loads
+  // wave (j / S) % W. A wave's first block is then known before the position is: its K/V loads
   // (clamped to the capacity, always valid memory) and the query loads go out at entry, and
   // the position read overlaps them.
   const int j0 = part + a.splits * w;
@@ -84,7 +89,7 @@ __global__ void __launch_bounds__(256) attn_kernel(AttnArgs a) {
     return *gmem(reinterpret_cast<const u32x4*>(qp));
   };
   if constexpr (QLDS) {
-    for (int i = w; i < RT * 4; i += 4) qlds[i * 64 + lane] = qload(i >> 2, i & 3);
+    for (int i = w; i < RT * 4; i += W) qlds[i * 64 + lane] = qload(i >> 2, i & 3);
     __syncthreads();
   } else {
 #pragma unroll
@@ -102,9 +107,9 @@ __global__ void __launch_bounds__(256) attn_kernel(AttnArgs a) {
   // Splits in use: at least one block per wave each (a short context on many splits would
   // only add partials and merge work). Workgroups past them leave now; when fewer splits
   // are used than launched, waves past the first fetch their first block again.
-  const int se = max(1, min(a.splits, (nblk + 3) >> 2));
+  const int se = live_splits(nblk, a.splits);
   if (part >= se) return;
-  const int j1 = part + se * w, jstep1 = 4 * se;
+  const int j1 = part + se * w, jstep1 = W * se;
   const int nb = j1 < nblk ? (nblk - j1 + jstep1 - 1) / jstep1 : 0;  // this wave's blocks
   if (PF && j1 != j0 && nb > 0) cur.load(kv, hb, 32 * j1, a.cap, n, g);
   // Last live key + 1 of row 16 rt + n (padding rows: every live key).
@@ -216,7 +221,7 @@ __global__ void __launch_bounds__(256) attn_kernel(AttnArgs a) {
     }
   }
 
-  // Merge the four waves: wave maxima and totals, then each wave's accumulator rescaled to
+  // Merge the waves: wave maxima and totals, then each wave's accumulator rescaled to
   // the workgroup maximum, summed over waves in order.
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
@@ -229,13 +234,19 @@ __global__ void __launch_bounds__(256) attn_kernel(AttnArgs a) {
     }
   }
   __syncthreads();
+  auto wg_max = [&](int r) {
+    float M = wm[0][r];
+#pragma unroll
+    for (int q = 1; q < W; ++q) M = fmaxf(M, wm[q][r]);
+    return M;
+  };
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = 16 * rt + 4 * g + i;
       if (r >= a.R) continue;
-      const float M = fmaxf(fmaxf(wm[0][r], wm[1][r]), fmaxf(wm[2][r], wm[3][r]));
+      const float M = wg_max(r);
       const float f = wm[w][r] == kNegInf ? 0.f : ex2(wm[w][r] - M);
       float* dst = wacc + ((size_t)w * a.R + r) * 128 + 8 * n;
       f32x4 lo, hi;
@@ -252,11 +263,11 @@ __global__ void __launch_bounds__(256) attn_kernel(AttnArgs a) {
 
   // Workgroup result per (row, 4 dims): maximum M, total L, accumulator A (waves in order).
   auto wg_result = [&](int r, int d4, float& M, float& L) -> f32x4 {
-    M = fmaxf(fmaxf(wm[0][r], wm[1][r]), fmaxf(wm[2][r], wm[3][r]));
+    M = wg_max(r);
     L = 0.f;
     f32x4 A = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < W; ++q) {
       const float f = wm[q][r] == kNegInf ? 0.f : ex2(wm[q][r] - M);
       L += wl[q][r] * f;
       A += *reinterpret_cast<const f32x4*>(wacc + ((size_t)q * a.R + r) * 128 + d4);
@@ -270,7 +281,7 @@ __global__ void __launch_bounds__(256) attn_kernel(AttnArgs a) {
   };
   const int items = a.R * 32;
   if (se == 1) {
-    for (int idx = threadIdx.x; idx < items; idx += 256) {
+    for (int idx = threadIdx.x; idx < items; idx += 64 * W) {
       const int r = idx >> 5, d4 = (idx & 31) * 4;
       float M, L;
       const f32x4 A = wg_result(r, d4, M, L);
@@ -284,7 +295,7 @@ __global__ void __launch_bounds__(256) attn_kernel(AttnArgs a) {
   // Partials: acc [heads][S][R][128], then maxima and totals [heads][S][R].
   const size_t pb = ((size_t)head * a.splits + part) * a.R;
   const size_t nslot = (size_t)a.heads * a.splits * a.R;
-  for (int idx = threadIdx.x; idx < items; idx += 256) {
+  for (int idx = threadIdx.x; idx < items; idx += 64 * W) {
     const int r = idx >> 5, d4 = (idx & 31) * 4;
     float M, L;
     const f32x4 A = wg_result(r, d4, M, L);
@@ -300,8 +311,8 @@ __global__ void __launch_bounds__(256) attn_kernel(AttnArgs a) {
 // x row: its loads spread over that many CUs, not one per head): the splits in use (se, from
 // the same position) combine as in attention.py:144-178 -- weights exp(max_s - max), weighted
 // accumulators over weighted totals -- in a fixed order. ng thread groups share an item's
-// splits (contiguous ranges); a thread issues the loads of up to 16 splits at once (one memory
-// round trip), merges them, and the groups' results combine in group order through LDS. With
+// splits (contiguous ranges); a thread issues the loads of 4 splits at once (32 splits: one
+// memory round trip; 16, mostly clamped repeats, took longer), merges them, and the groups' results combine in group order through LDS. With
 // one split in use the attention kernel wrote the output itself.
 __global__ void __launch_bounds__(256) attn_merge_kernel(AttnArgs a) {
   extern __shared__ float gbuf[];  // the groups' results: 6 floats per slot
@@ -311,7 +322,7 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(AttnArgs a) {
   const int base = __builtin_amdgcn_readfirstlane(a.pos[0]);
   const int end = min(base + a.T, a.cap);
   const int nblk = end > 0 ? (end + 31) >> 5 : 0;
-  const int se = max(1, min(a.splits, (nblk + 3) >> 2));
+  const int se = live_splits(nblk, a.splits);
   if (se == 1) return;
   const int items = 32, row = blockIdx.y;  // items: the row's 4-value chunks
   const int ng = 256 / items;
@@ -329,11 +340,11 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(AttnArgs a) {
     const int s_lo = sg * per, s_hi = min(se, s_lo + per);
     float Mt = kNegInf, Lt = 0.f;
     f32x4 At = {0.f, 0.f, 0.f, 0.f};
-    for (int b0 = s_lo; b0 < s_hi; b0 += 16) {
-      float mv[16], lv[16];
-      f32x4 av[16];
+    for (int b0 = s_lo; b0 < s_hi; b0 += 4) {
+      float mv[4], lv[4];
+      f32x4 av[4];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
+      for (int j = 0; j < 4; ++j) {
         const size_t o = hb0 + (size_t)min(b0 + j, s_hi - 1) * a.R + r;
         mv[j] = gmem(P)[nslot * 128 + o];
         lv[j] = gmem(P)[nslot * 129 + o];
@@ -341,14 +352,14 @@ __global__ void __launch_bounds__(256) attn_merge_kernel(AttnArgs a) {
       }
       float Mb = Mt;
 #pragma unroll
-      for (int j = 0; j < 16; ++j)
+      for (int j = 0; j < 4; ++j)
         if (b0 + j < s_hi) Mb = fmaxf(Mb, mv[j]);
       const float Mu = Mb == kNegInf ? 0.f : Mb;
       const float c = Mt == kNegInf ? 0.f : ex2(Mt - Mu);
       At *= c;
       Lt *= c;
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
+      for (int j = 0; j < 4; ++j) {
         if (b0 + j >= s_hi || mv[j] == kNegInf) continue;
         const float f = ex2(mv[j] - Mu);
         At += f * av[j];

@@ -37,7 +37,7 @@ typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 __device__ __forceinline__ bf16x8 bf8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
 __device__ __forceinline__ uint32_t pack_bf(float lo, float hi) {
-  return (uint32_t)f2bf(lo) | ((uint32_t)f2bf(hi) << 16);
+  return bf16_canonical_nan(bf16_pair_hw(lo, hi));
 }
 
 template <bool Q8>
@@ -114,23 +114,24 @@ struct KVBlock<true> {
         vsc[j] = 0.f;
       }
   }
-  static __device__ __forceinline__ float deq(uint32_t w, int b, float sc) {
-    return round_bf((float)(int)(int8_t)(w >> (8 * b)) * sc);
+  // bf16(code * scale) of two codes, bytes b0 of w0 and b1 of w1: the hardware's pair conversion (a
+  // product rounded value by value, then packed by rounding again, was 16 instructions a value and
+  // most of the kernel: 40 MB of cache at batch 32, 577 keys, 33.2 us; 2.5 instructions this way).
+  static __device__ __forceinline__ uint32_t deq2(uint32_t w0, int b0, float s0, uint32_t w1, int b1, float s1) {
+    return bf16_pair_hw((float)(int)(int8_t)(w0 >> (8 * b0)) * s0, (float)(int)(int8_t)(w1 >> (8 * b1)) * s1);
   }
   __device__ __forceinline__ u32x4 kfrag(int kt, int s) const {
     const uint32_t* c = reinterpret_cast<const uint32_t*>(&k[kt][s >> 1]) + 2 * (s & 1);
     const float sc = ksc[kt];
-    return u32x4{pack_bf(deq(c[0], 0, sc), deq(c[0], 1, sc)), pack_bf(deq(c[0], 2, sc), deq(c[0], 3, sc)),
-                 pack_bf(deq(c[1], 0, sc), deq(c[1], 1, sc)), pack_bf(deq(c[1], 2, sc), deq(c[1], 3, sc))};
+    return u32x4{deq2(c[0], 0, sc, c[0], 1, sc), deq2(c[0], 2, sc, c[0], 3, sc), deq2(c[1], 0, sc, c[1], 1, sc),
+                 deq2(c[1], 2, sc, c[1], 3, sc)};
   }
   __device__ __forceinline__ u32x4 vfrag(int c) const {
     uint32_t d[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint32_t w0 = reinterpret_cast<const uint32_t*>(&v[2 * q])[c >> 2];
-      const uint32_t w1 = reinterpret_cast<const uint32_t*>(&v[2 * q + 1])[c >> 2];
-      d[q] = pack_bf(deq(w0, c & 3, vsc[2 * q]), deq(w1, c & 3, vsc[2 * q + 1]));
-    }
+    for (int q = 0; q < 4; ++q)
+      d[q] = deq2(reinterpret_cast<const uint32_t*>(&v[2 * q])[c >> 2], c & 3, vsc[2 * q],
+                  reinterpret_cast<const uint32_t*>(&v[2 * q + 1])[c >> 2], c & 3, vsc[2 * q + 1]);
     return u32x4{d[0], d[1], d[2], d[3]};
   }
 };
