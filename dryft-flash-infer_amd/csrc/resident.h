@@ -4,13 +4,17 @@
 // every 1 KB of 8-bit weights and 16 tokens, 4 KB for 4-bit ones), after a pass that stages the
 // activation and a barrier, and run the code-bias chain beside the main one. Here a wave keeps one
 // K range for the whole launch, so its activation fragments and code-bias totals stay in registers:
-//   * a workgroup of 8 waves owns one K slice and a run of 16-row tiles; wave w holds units
-//     w U .. w U + U - 1 of the slice (a unit is 1 KB of a tile: one 16-byte load per lane, 128 k
-//     of 4-bit or 64 k of 8-bit codes) and streams those units of every tile of the run, D tiles
+//   * a workgroup of 8 waves owns one K slice and a run of 16-row tiles; the slice's units go to
+//     the waves evenly, at most U each (a unit is 1 KB of a tile: one 16-byte load per lane, 128 k
+//     of 4-bit or 64 k of 8-bit codes). A wave streams its units of every tile of the run, D tiles
 //     ahead of its MFMAs. Weights go from memory through registers into MFMAs; nothing else is
 //     read per tile but the scales;
-//   * the 8 partial sums of a tile meet in LDS (double buffered, one barrier per tile), one wave
-//     adds them in wave order and writes the output; waves take turns;
+//   * the activation is loaded in memory order and turned into fragments through LDS, unit by
+//     unit, while the first weights are on their way. This start is what bounds the calls of many
+//     tokens: 2560 x 19456 W4A16 at 64 tokens 19.3 us with loads in fragment order, 18.0 now;
+//     4096 x 2560 W8A16 at 32 tokens 9.5 and 9.1 (in one slice 12.3 and 9.3);
+//   * the 8 partial sums of D tiles meet in LDS (two sets, one barrier per D tiles); every wave
+//     adds its part of them in wave order and writes outputs;
 //   * K slices (where one slice does not fit the registers, or the tiles do not fill the CUs) write
 //     fp32 planes that the run's last workgroup sums in slice order;
 //   * 33..64 tokens run as two blocks of 32, ids 8 apart (one XCD), the second reading the weights
@@ -122,12 +126,6 @@ __device__ __forceinline__ void transpose_rows(uint32_t (&a)[4]) {
   }
 }
 
-// The value of lane + N of the lane's group of 16 (past it: 0).
-template <int N>
-__device__ __forceinline__ uint32_t row_shl(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x100 + N, 0xf, 0xf, false);
-}
-
 // What each of the four lane groups of 16 holds in v, to all of them: out[i] = group i's value.
 __device__ __forceinline__ void spread_groups(uint32_t v, uint32_t* out) {
   const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);  // {0, 1, 0, 1}, {2, 3, 2, 3}
@@ -169,46 +167,29 @@ __device__ __forceinline__ f32x4 mfma_fp8(const uint4& a, const uint4& b, f32x4 
                                                     (long)(((unsigned long)b.w << 32) | b.z), c, 0, 0, 0);
 }
 
-// The fragments of a unit as loaded (fragment t of lane group c: bytes 64 t + 16 c of the unit's
-// row, so that 4 lanes read 64 consecutive bytes) into the order in which the codes unpack.
+// The 16-byte chunk of a unit's row that lane group c reads as its fragment t. The reference formats
+// take dwords from all chunks of a block (unit_order).
+template <class F>
+__device__ __forceinline__ int frag_chunk(int c, int t) {
+  return is_ref<F>() ? 4 * t + c : Unit<F>::NF * c + t;
+}
+// A unit's fragments into the order in which the codes unpack.
 template <class F>
 __device__ __forceinline__ void unit_order(uint4 (&f)[Unit<F>::NF]) {
-  uint32_t d[Unit<F>::NF][4];
-#pragma unroll
-  for (int t = 0; t < Unit<F>::NF; ++t) d[t][0] = f[t].x, d[t][1] = f[t].y, d[t][2] = f[t].z, d[t][3] = f[t].w;
-  if constexpr (std::is_same<F, FmtW4>::value) {
-    // lane group c takes values 32 c .. + 31: pieces 4 c + t of the row's 16
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      uint32_t p[4] = {d[0][e], d[1][e], d[2][e], d[3][e]};
-      transpose_rows(p);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) d[t][e] = p[t];
-    }
-  } else if constexpr (std::is_same<F, FmtW8>::value) {
-    // lane group c takes values 16 c .. + 15: pieces 2 c + t of the row's 8
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      auto v = __builtin_amdgcn_permlane32_swap(d[0][e], d[1][e], false, false);
-      v = __builtin_amdgcn_permlane16_swap(v[0], v[1], false, false);
-      d[0][e] = v[0], d[1][e] = v[1];
-    }
-  } else {
-    // The reference's permutation: lane group c of a 64-value block takes the pairs 16 s + 2 c and
-    // 16 s + 2 c + 8 of every s (FmtRef::stage_chunk), dword c of each of the block's 8 pieces.
-#pragma unroll
-    for (int t = 0; t < Unit<F>::NF; ++t) transpose_rows(d[t]);
-  }
 #pragma unroll
   for (int t = 0; t < Unit<F>::NF; ++t) {
-    const uint4 v = {d[t][0], d[t][1], d[t][2], d[t][3]};
-    if constexpr (std::is_same<F, FmtRef<4>>::value)
-      f[t] = uint4{__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.y, v.x, 0x07060302u),
-                   __builtin_amdgcn_perm(v.w, v.z, 0x05040100u), __builtin_amdgcn_perm(v.w, v.z, 0x07060302u)};
-    else if constexpr (std::is_same<F, FmtRef<8>>::value)
-      f[t] = v;
-    else
-      f[t] = F::order(v);
+    if constexpr (is_ref<F>()) {
+      // The reference's permutation: lane group c of a 64-value block takes the pairs 16 s + 2 c and
+      // 16 s + 2 c + 8 of every s (FmtRef::stage_chunk), dword c of each of the block's 8 chunks.
+      uint32_t d[4] = {f[t].x, f[t].y, f[t].z, f[t].w};
+      transpose_rows(d);
+      f[t] = uint4{d[0], d[1], d[2], d[3]};
+      if constexpr (std::is_same<F, FmtRef<4>>::value)
+        f[t] = uint4{__builtin_amdgcn_perm(d[1], d[0], 0x05040100u), __builtin_amdgcn_perm(d[1], d[0], 0x07060302u),
+                     __builtin_amdgcn_perm(d[3], d[2], 0x05040100u), __builtin_amdgcn_perm(d[3], d[2], 0x07060302u)};
+    } else {
+      f[t] = F::order(f[t]);
+    }
   }
 }
 
@@ -286,6 +267,14 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) r
       else sb[d][0] = __builtin_amdgcn_raw_buffer_load_b16(sr, (int)at.sc, 0, 0);
     }
   };
+  // Activations are loaded in memory order -- load t: ROWS token rows of the unit, 16 bytes a lane along
+  // a row -- and turned into fragments (lane r: token r) through the wave's part of the second set of
+  // partial sums, idle until the first barrier. (Loads in fragment order, consecutive lanes in
+  // consecutive rows, take the CU 4 times as long: 160 KB by 8 waves 4.6 us, in memory order 1.7.)
+  // Slots of a row lie rotated by its index (exclusive or), so that reads hit every bank alike.
+  constexpr int CH = 4 * NF, ROWS = 16 / NF, NL = FEW ? 1 : NF;  // 16-byte chunks of a row; rows, loads
+  uint4* const turn = reinterpret_cast<uint4*>(red + 8 * P * 256) + wave * (64 * NL);
+  const unsigned xoff = (unsigned)(lane / CH) * (unsigned)a.k * XB + (unsigned)(lane % CH) * 16u;
   // Unit by unit its weights of the first D tiles, then its activation fragments: the order in which
   // the first block needs them, memory's requests before the cache's.
   {
@@ -298,19 +287,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) r
     for (int u = 0; u < U; ++u) {
 #pragma unroll
       for (int d = 0; d < D; ++d) load_unit(d, u, at[d]);
-      if constexpr (FEW) {  // lane r loads fragment r / (16 / NF) of token r % (16 / NF)
-        const unsigned off = (unsigned)(r % (16 / NF)) * (unsigned)a.k * XB + (unsigned)(c * 16 + r / (16 / NF) * 64);
-        xf[u][0][0] = resident_load16(xr, off | idle[u], (u0 + u) * (UT::KV * XB));
-        continue;
-      }
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        // rows past the tokens lie past the buffer: zeros
-        const unsigned off = (unsigned)(16 * mt + r) * (unsigned)a.k * XB + (unsigned)(c * 16);
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int t = 0; t < NF; ++t)
-          xf[u][mt][t] = resident_load16(xr, (off + 64u * t) | idle[u], (u0 + u) * (UT::KV * XB));
-      }
+        for (int t = 0; t < NL; ++t)  // rows past the tokens lie past the buffer: zeros
+          xf[u][mt][t] = resident_load16(xr, (xoff + (unsigned)(16 * mt + t * ROWS) * (unsigned)a.k * XB) | idle[u],
+                                         (u0 + u) * (UT::KV * XB));
     }
   }
   // Code-bias totals: the main chain with every code at the bias, so that a zero weight cancels
@@ -352,27 +334,25 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) r
       for (int mt = 0; mt < MT; ++mt) acc[d][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
     // Activation fragments of unit u into the codes' order, and its bias totals (first block only).
     auto ready_unit = [&](int u) __attribute__((always_inline)) {
-      if constexpr (FP8) return;
-      else {
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        if constexpr (FEW) {
-          // fragment t of token r comes from lane r + 16 / NF * t; lanes past the tokens get
-          // other fragments, whose products land in rows that are dropped
-          static_for<1, NF>([&](auto tc) __attribute__((always_inline)) {
-            constexpr int t = decltype(tc)::value;
-            const uint4 v = xf[u][0][0];
-            xf[u][0][t] = uint4{row_shl<16 / NF * t>(v.x), row_shl<16 / NF * t>(v.y), row_shl<16 / NF * t>(v.z),
-                                row_shl<16 / NF * t>(v.w)};
-          });
-        }
-        unit_order<F>(xf[u][mt]);
 #pragma unroll
-        for (int t = 0; t < NF; ++t) {
-          f32x4& b = tb[NG ? u : 0][NG ? t / PER : 0][mt];
-          b = mfma_bf16(xf[u][mt][t], bias, b);
+        for (int t = 0; t < NL; ++t) {
+          const int row = t * ROWS + lane / CH;
+          turn[row * CH + ((lane % CH) ^ (row / (16 / CH)))] = xf[u][mt][t];
         }
-      }
+        const int row = FEW ? r % ROWS : r;  // rows past the tokens: others', whose products are dropped
+#pragma unroll
+        for (int t = 0; t < NF; ++t)
+          xf[u][mt][t] = turn[row * CH + (frag_chunk<F>(c, t) ^ (row / (16 / CH)))];
+        if constexpr (!FP8) {
+          unit_order<F>(xf[u][mt]);
+#pragma unroll
+          for (int t = 0; t < NF; ++t) {
+            f32x4& b = tb[NG ? u : 0][NG ? t / PER : 0][mt];
+            b = mfma_bf16(xf[u][mt][t], bias, b);
+          }
+        }
       }
     };
     auto multiply = [&](int d, int u) __attribute__((always_inline)) {
@@ -525,7 +505,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) r
 
 template <class F, int MT, int U, int D, bool FEW>
 hipError_t resident_launch(const ResidentArgs& a, hipStream_t st) {
-  constexpr int lds = 2 * 8 * D * MT * 1024;
+  constexpr int sums = 8 * D * MT * 1024, turn = 8 * (FEW ? 1 : Unit<F>::NF) * 1024;
+  constexpr int lds = sums + (sums > turn ? sums : turn);
   static_assert(lds <= 128 * 1024, "partial sums");
   if (lds > 64 * 1024) {
     static int allowed = 64 * 1024;
