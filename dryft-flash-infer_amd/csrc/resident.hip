@@ -4,10 +4,12 @@
 namespace qlx {
 
 // K slices of a shape, 0 where the kernel does not serve it: the least of a time in microseconds,
-// fitted to a sweep of 1 to 8 slices over the Qwen3-4B projections in all five formats at 1, 4, 8, 16,
-// 32 and 64 tokens (MI355X). A CU takes in about 40 KB of weights or activations per microsecond, the
-// weights of the whole call come at 5.6 TB/s; slices cost their planes, a ticket and a round trip for
-// the sum.
+// fitted to a sweep of 1 to 8 slices over the Qwen3-4B projections in all five formats at 1 to 64
+// tokens and over 70 other shapes (n 960 to 24000, k 1024 to 13824; MI355X). A CU takes in about 25 KB
+// of weights and 40 of activations per microsecond, the weights of the whole call come at 5.6 TB/s;
+// slices cost their planes, a ticket and a round trip for the sum. The slices it picks take 0.3 % more
+// time than the best of the eight on the Qwen3-4B projections, 1.1 % on the others (W8A16 down: 12.3
+// -> 11.6 us at 24 tokens, 16.5 -> 14.3 at 64 against an earlier fit, which was 1.4 and 1.7 % off).
 template <class F>
 int resident_splits(int m, int n, int k) {
   const int units = k / Unit<F>::KV, ntiles = n / 16, rows = std::min(m, 32);
@@ -17,10 +19,10 @@ int resident_splits(int m, int n, int k) {
     ResidentPlan p;
     if (!resident_plan<F>(m, n, k, s, p) || p.splits != s) continue;
     const int tiles = (ntiles + p.groups - 1) / p.groups;
-    const double weights = std::max((double)ntiles * units / 5600, (double)tiles * p.per_slice / 30);
+    const double weights = std::max((double)ntiles * units / 5600, (double)tiles * p.per_slice / 25);
     const double acts = rows * (double)p.per_slice * (Unit<F>::KV * F::XBYTES / 1024.0) / 40;
     const int rounds = (tiles * 4 * rows + 511) / 512, depth = resident_depth<F>(rows > 16 ? 2 : 1, p.u);
-    const double slices = s > 1 ? 1.2 + 0.8 * rounds + 0.12 * s + (double)s * m * n * 8 / 4e6 : 0;
+    const double slices = s > 1 ? 0.8 + 1.2 * rounds + 0.2 * s + (double)s * m * n * 8 / 2e6 : 0;
     const double t = weights + acts + slices + 0.5 * std::min((tiles + depth - 1) / depth - 1, 2);
     if (best == 0 || t < least) best = s, least = t;
   }
