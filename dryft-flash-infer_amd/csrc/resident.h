@@ -254,16 +254,20 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) r
   // unit's weights.
   constexpr int SQ = NG ? (U + 3) / 4 : 1;
   uint32_t sb[D][SQ];
+  // Scalar offsets stay inside their buffer for units past the slice too (a wave of a short last slice
+  // may hold several fewer than U): whether a load is in range is decided by the lane offset alone.
+  const int last_unit = a.units - 1;
   auto load_unit = [&](int d, int u, const At& at) __attribute__((always_inline)) {
-    const int uu = u0 + u;
+    const int uu = min(u0 + u, last_unit);
     wb[d][u] = resident_load16(wr, at.w | idle[u], std::is_same<F, FmtRef<8>>::value ? (uu >> 1) * 2048 + (uu & 1) * 512 : uu * 1024);
   };
+  const int su = min(u0, last_unit);
   auto load_scales = [&](int d, const At& at) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < SQ; ++q) {
       const unsigned off = at.sc | (4 * q + c < held ? 0u : kOutOfRange);
-      if constexpr (NG == 1) sb[d][q] = __builtin_amdgcn_raw_buffer_load_b16(sr, (int)(off + 2 * (4 * q + c)), u0 * 2, 0);
-      else if constexpr (NG == 2) sb[d][q] = __builtin_amdgcn_raw_buffer_load_b32(sr, (int)(off + 4 * (4 * q + c)), u0 * 4, 0);
+      if constexpr (NG == 1) sb[d][q] = __builtin_amdgcn_raw_buffer_load_b16(sr, (int)(off + 2 * (4 * q + c)), su * 2, 0);
+      else if constexpr (NG == 2) sb[d][q] = __builtin_amdgcn_raw_buffer_load_b32(sr, (int)(off + 4 * (4 * q + c)), su * 4, 0);
       else sb[d][0] = __builtin_amdgcn_raw_buffer_load_b16(sr, (int)at.sc, 0, 0);
     }
   };
@@ -292,7 +296,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) r
 #pragma unroll
         for (int t = 0; t < NL; ++t)  // rows past the tokens lie past the buffer: zeros
           xf[u][mt][t] = resident_load16(xr, (xoff + (unsigned)(16 * mt + t * ROWS) * (unsigned)a.k * XB) | idle[u],
-                                         (u0 + u) * (UT::KV * XB));
+                                         min(u0 + u, last_unit) * (UT::KV * XB));
     }
   }
   // Code-bias totals: the main chain with every code at the bias, so that a zero weight cancels

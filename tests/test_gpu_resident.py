@@ -179,3 +179,12 @@ def test_graph_replays_equal_eager():
         torch.cuda.synchronize()
         assert torch.equal(out, cuda_fp8.matmul(x, p))
     assert eager.shape == out.shape
+
+
+@pytest.mark.parametrize("fmt,k,splits", [("w4a16", 8448, 4), ("fp8", 3328, 6), ("int4g64", 8448, 4)])
+def test_a_short_last_slice_of_one_token(fmt, k, splits):
+    """A last K slice whose waves hold several units fewer than the others', the last of them at the end
+    of the weight (one tile) and of the activation (one token)."""
+    p = make(fmt, 16, k, 61)[1]
+    x = acts(1, k, 62)
+    close(resident(fmt, x, p, splits), decode(fmt, x, p, False), False, (fmt, k, splits))
