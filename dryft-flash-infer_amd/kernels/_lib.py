@@ -7,6 +7,7 @@ run time. There is no fallback: without the library every op raises.
 """
 
 import ctypes
+import itertools
 import os
 
 import torch  # noqa: F401  (loads the HIP runtime the library then shares)
@@ -213,3 +214,26 @@ def tickets(device, count):
         buf = torch.zeros(size, dtype=torch.int32, device=device)
         _tickets[index] = buf
     return buf
+
+
+#: Counters of one stream's slot and slots of a device (64 x 2 KB).
+STREAM_TICKETS = 512
+STREAM_SLOTS = 64
+_stream_tickets = {}
+
+
+def stream_tickets(device, stream):
+    """The address of ``STREAM_TICKETS`` zeroed counters for one stream's split-K calls: calls that
+    overlap on different streams count apart (from the 65th stream on, slots are shared in turn)."""
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    pool = _stream_tickets.get(index)
+    if pool is None:
+        buf = torch.zeros(STREAM_SLOTS * STREAM_TICKETS, dtype=torch.int32, device=device)
+        if not torch.cuda.is_current_stream_capturing():  # once: other streams' first calls find it zeroed
+            torch.cuda.current_stream(device).synchronize()
+        pool = _stream_tickets.setdefault(index, (buf, {}, itertools.count()))
+    buf, slots, count = pool
+    slot = slots.get(stream)
+    if slot is None:
+        slot = slots.setdefault(stream, next(count) % STREAM_SLOTS)
+    return buf.data_ptr() + slot * STREAM_TICKETS * 4

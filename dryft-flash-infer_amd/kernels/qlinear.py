@@ -214,6 +214,7 @@ def run_resident(plan, fmt, q, s, x, xs, m, n, k):
     """``qlx_linear_resident`` with ``plan``: bf16 ``[m, n]`` (SwiGLU ``[m, n/2]``), or fp32 planes
     ``[splits, m, n]`` where the plan's mode is planes."""
     device = x.device
+    stream = _lib.stream(device)
     planes = plan.mode == _lib.MODE_PLANES
     work = out = None
     if x.data_ptr() % 16:  # the kernel reads it in 16-byte pieces
@@ -224,9 +225,9 @@ def run_resident(plan, fmt, q, s, x, xs, m, n, k):
     if not planes:
         out = torch.empty((m, n // 2 if plan.mode == _lib.MODE_SWIGLU else n), dtype=torch.bfloat16, device=device)
         if plan.splits > 1:
-            plan.tickets = _lib.tickets(device, 512).data_ptr()
+            plan.tickets = _lib.stream_tickets(device, stream)
     _lib.call("qlx_linear_resident", fmt, _lib.ptr(q), _lib.ptr(s), _lib.ptr(x), _lib.ptr(xs), _lib.ptr(out), m, n, k,
-              ctypes.byref(plan), _lib.stream(device))
+              ctypes.byref(plan), stream)
     return work if planes else out
 
 

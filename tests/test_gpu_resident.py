@@ -86,7 +86,7 @@ def test_resident_matches_decode_kernel(fmt, n, k, swiglu):
             if not swiglu:
                 assert not got[:, 0].float().abs().sum().item(), "a zero weight row gives zero"
         assert served or (m > 32 and n < 128), (fmt, n, k, m)
-    assert int(_lib.tickets(torch.device(DEV), 512)[:512].abs().sum()) == 0, "tickets are left at zero"
+    assert all(int(buf.abs().sum()) == 0 for buf, _, _ in _lib._stream_tickets.values()), "tickets are left at zero"
 
 
 @pytest.mark.parametrize("fmt", list(FMTS))
@@ -179,6 +179,29 @@ def test_graph_replays_equal_eager():
         torch.cuda.synchronize()
         assert torch.equal(out, cuda_fp8.matmul(x, p))
     assert eager.shape == out.shape
+
+
+def test_calls_of_two_streams_count_apart():
+    """K slices' tickets: a slot per stream, the same on the next call; overlapping calls' results are
+    those of the calls one after the other."""
+    fmt, m, n, k = "w8a16", 8, 2560, 9728
+    ps = [make(fmt, n, k, seed)[1] for seed in (51, 52)]
+    xs = [acts(m, k, seed) for seed in (53, 54)]
+    want = [bits16(resident(fmt, x, p, 4)) for x, p in zip(xs, ps)]
+    streams = [torch.cuda.Stream(DEV) for _ in range(2)]
+    slots = [_lib.stream_tickets(torch.device(DEV), st.cuda_stream) for st in streams]
+    assert abs(slots[0] - slots[1]) >= 4 * _lib.STREAM_TICKETS
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(8):
+        for i, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                got[i].append(resident(fmt, xs[i], ps[i], 4))
+    torch.cuda.synchronize()
+    assert slots == [_lib.stream_tickets(torch.device(DEV), st.cuda_stream) for st in streams]
+    for i in range(2):
+        for y in got[i]:
+            assert (bits16(y) == want[i]).all()
 
 
 @pytest.mark.parametrize("fmt,k,splits", [("w4a16", 8448, 4), ("fp8", 3328, 6), ("int4g64", 8448, 4)])
