@@ -312,8 +312,9 @@ __global__ void __launch_bounds__(64 * W) attn_kernel(AttnArgs a) {
 // the same position) combine as in attention.py:144-178 -- weights exp(max_s - max), weighted
 // accumulators over weighted totals -- in a fixed order. ng thread groups share an item's
 // splits (contiguous ranges); a thread issues the loads of 4 splits at once (32 splits: one
-// memory round trip; 16, mostly clamped repeats, took longer), merges them, and the groups' results combine in group order through LDS. With
-// one split in use the attention kernel wrote the output itself.
+// memory round trip; 16, mostly clamped repeats, took longer), merges them, and the groups'
+// results combine in group order through LDS. With one split in use the attention kernel wrote
+// the output itself.
 __global__ void __launch_bounds__(256) attn_merge_kernel(AttnArgs a) {
   extern __shared__ float gbuf[];  // the groups' results: 6 floats per slot
   const int head = blockIdx.x;

@@ -4,9 +4,9 @@
 //   scale = 1 / sqrt(mean(x^2) + eps)          (fp32; the sum of squares exact in fp64)
 //   n     = bf16(bf16(x * scale) * w)
 //   y     = bf16(bf16(n * cos) + bf16(rotate_half(n) * sin)),  rotate_half(n) = (-n[64:], n[:64])
-// Eight lanes per 128-value head: lane j holds dims 8 j .. 8 j + 7 and their rotate_half partners
-// 64 + 8 j .. 64 + 8 j + 7, so the rotation stays in the lane and only the sum of squares
-// crosses lanes (shuffles among the 8 lanes of a head).
+// Sixteen lanes per 128-value head (rope.hip; eight in the executor's stage): lane j holds dims
+// N j .. N j + N - 1 (N = 4; 8) and their rotate_half partners 64 dims on, so the rotation stays in
+// the lane and only the sum of squares crosses lanes (shuffles among a head's lanes).
 #pragma once
 
 #include "common.h"

@@ -27,8 +27,8 @@ The same signatures also carry the MI355X north-star formats, so an engine that 
   ``FormatPrepared`` with the attributes the engine reads (``bits``, ``k``, ``rows``,
   ``bytes_moved()``);
 * the linears dispatch on it: ``matmul``/``gate_up_swiglu`` take the library's planned
-  path for the batch (the resident-activation GEMM where its plan has the call, else decode kernel or skinny GEMM; FP8 activation quantized
-  once from 2 tokens), ``matmul_partials``/``splits`` honour the config's split-K.
+  path for the batch (the resident-activation GEMM where its plan has the call, else decode
+  kernel or skinny GEMM; FP8 activation quantized once from 2 tokens), ``matmul_partials``/``splits`` honour the config's split-K.
 """
 
 import os
