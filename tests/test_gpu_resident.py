@@ -2,9 +2,9 @@
 token fragments and blocks (1 to 64 tokens), one tile to more tiles than workgroups, waves without
 units, each K-slice count the shape takes, SwiGLU halves that are not whole tiles.
 
-The checker is the decode kernel on the same weights (the same products summed in another order, so
+The comparison is with the decode kernel on the same weights (the same products summed in another order, so
 outputs within one bf16 rounding step: 2^-7 of the value plus 2^-9 of the row's largest; SwiGLU, two
-roundings more, 2^-6), and the oracle's dequantize-then-matmul at the north star's rel-L2 of 1e-2. A
+roundings more, 2^-6), and the oracle's dequantize-then-matmul at a rel-L2 of 1e-2. A
 zero weight row gives exactly zero; fp32 planes summed in slice order are the reduced output."""
 
 import numpy as np
