@@ -574,6 +574,17 @@ bool resident_plan(int m, int n, int k, int splits, ResidentPlan& p) {
   return true;
 }
 
+// Why the kernel cannot take a call of these sizes in `splits` K slices, nullptr where it can: its
+// offsets within each operand are 32 bits, the top one of them the sign of a load out of range.
+template <class F>
+const char* resident_limit(int m, int n, int k, int splits) {
+  constexpr long long most = 1ll << 31;
+  if ((long long)(n / 16) * (k / Unit<F>::KV) * 1024 >= most) return "weights of under 2 GiB";
+  if ((long long)std::min(m, 32) * k * F::XBYTES >= most) return "activations of under 2 GiB";
+  if ((long long)splits * m * n * 4 >= most) return "planes of under 2 GiB";
+  return nullptr;
+}
+
 template <class F>
 int resident_run(const char* name, ResidentArgs a, int m, int n, int k, const qlx_plan* plan, void* stream) {
   QLX_REQUIRE(plan != nullptr, "%s: plan is NULL", name);
@@ -581,21 +592,21 @@ int resident_run(const char* name, ResidentArgs a, int m, int n, int k, const ql
   QLX_REQUIRE(n >= 16 && n % 16 == 0 && k >= 128 && k % 128 == 0 && k % F::KSTEP == 0,
               "%s: n=%d k=%d do not fit the tiled format", name, n, k);
   QLX_REQUIRE(plan->mode >= QLX_MODE_BF16 && plan->mode <= QLX_MODE_SWIGLU, "%s: mode %d", name, plan->mode);
-  // 16-byte buffer loads of weights and activations, 4-byte ones of scales
-  QLX_REQUIRE(((uintptr_t)a.w | (uintptr_t)a.x) % 16 == 0 && ((uintptr_t)a.ws | (uintptr_t)a.y) % 4 == 0,
-              "%s: operands must start on 16-byte boundaries (scales, outputs: 4)", name);
   const int units = k / Unit<F>::KV;
-  QLX_REQUIRE((long long)(n / 16) * units * 1024 < (1ll << 31), "%s: weights of under 2 GiB (n=%d k=%d)", name, n, k);
   QLX_REQUIRE(plan->splits >= 1 && plan->splits <= units, "%s: splits must be 1..%d", name, units);
   ResidentPlan p;
   QLX_REQUIRE(resident_plan<F>(m, n, k, plan->splits, p), "%s: %d K slices leave a wave more than %d units", name,
               plan->splits, resident_max_units<F>(m <= 16 ? 1 : 2));
+  const char* const limit = resident_limit<F>(m, n, k, p.splits);
+  QLX_REQUIRE(limit == nullptr, "%s: %s (m=%d n=%d k=%d, %d slices)", name, limit, m, n, k, p.splits);
+  // 16-byte buffer loads of weights and activations, 4-byte ones of scales
+  QLX_REQUIRE(((uintptr_t)a.w | (uintptr_t)a.x) % 16 == 0 && ((uintptr_t)a.ws | (uintptr_t)a.y) % 4 == 0,
+              "%s: operands must start on 16-byte boundaries (scales, outputs: 4)", name);
   const bool planes = plan->mode == QLX_MODE_PLANES;
   QLX_REQUIRE(!planes || p.splits == plan->splits, "%s: %d splits leave %d non-empty planes", name, plan->splits, p.splits);
   QLX_REQUIRE(planes ? plan->workspace != nullptr
                      : p.splits == 1 || (plan->workspace != nullptr && plan->tickets != nullptr),
               "%s: K slices need a workspace and tickets, planes a workspace", name);
-  QLX_REQUIRE((long long)p.splits * m * n * 4 < (1ll << 31), "%s: planes of under 2 GiB", name);
   a.m = m, a.n = n, a.k = k, a.half = n / 2, a.swiglu = plan->mode == QLX_MODE_SWIGLU;
   a.units = units, a.per_slice = p.per_slice, a.splits = p.splits;
   a.ntiles = n / 16, a.groups = p.groups, a.tblocks = p.tblocks;

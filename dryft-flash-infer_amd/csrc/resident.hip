@@ -17,7 +17,7 @@ int resident_splits(int m, int n, int k) {
   double least = 0;
   for (int s = 1; s <= 8 && s <= units; ++s) {
     ResidentPlan p;
-    if (!resident_plan<F>(m, n, k, s, p) || p.splits != s) continue;
+    if (!resident_plan<F>(m, n, k, s, p) || p.splits != s || resident_limit<F>(m, n, k, s)) continue;
     const int tiles = (ntiles + p.groups - 1) / p.groups;
     const double weights = std::max((double)ntiles * units / 5600, (double)tiles * p.per_slice / 25);
     const double acts = rows * (double)p.per_slice * (Unit<F>::KV * F::XBYTES / 1024.0) / 40;

@@ -184,9 +184,9 @@ int qlx_linear_skinny_fp8(const void* w, const void* w_scale, const void* x_code
  * in registers for the whole launch and streams that range of a run of 16-row weight tiles. FP8
  * takes the activation quantized beforehand (e4m3 codes, x_scale fp32 [m]); the others bf16 x and
  * no x_scale. Output bf16, SwiGLU, or the fp32 planes themselves (QLX_MODE_PLANES, in plan->workspace,
- * y unused); weights of under 2 GiB; w and x on 16-byte boundaries. qlx_plan_resident
- * fills plan->splits: 0 where no slice count fits the registers or another kernel measured faster
- * (qlx_linear_* / qlx_linear_skinny* serve those calls). With splits > 1 the call takes a workspace
+ * y unused); weights and planes of under 2 GiB each; w and x on 16-byte boundaries. qlx_plan_resident
+ * fills plan->splits: 0 where no slice count fits the registers and those sizes, or another kernel
+ * measured faster (qlx_linear_* / qlx_linear_skinny* serve those calls). With splits > 1 the call takes a workspace
  * of splits * m * n floats and 512 zeroed tickets (zero again afterwards). */
 int qlx_plan_resident(int fmt, int mode, int m, int n, int k, qlx_plan* plan);
 int qlx_linear_resident(int fmt, const void* w, const void* w_scale, const void* x, const float* x_scale, void* y,
