@@ -158,3 +158,14 @@ extern "C" int qlx_plan_fit(qlx_plan* plan, int fmt, int m, int n, int k, int co
   plan->splits = a.splits;
   return QLX_OK;
 }
+
+// The capture that a stream is in (0: none), the same for every stream that the capture has forked to.
+extern "C" int qlx_stream_capture(void* stream, unsigned long long* id) {
+  QLX_REQUIRE(id != nullptr, "stream_capture: id is NULL");
+  *id = 0;
+  if (stream == nullptr) return QLX_OK;  // the default stream cannot be captured
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  const hipError_t e = hipStreamGetCaptureInfo((hipStream_t)stream, &status, id);
+  if (status == hipStreamCaptureStatusNone) *id = 0;
+  return qlx::hip_status(e, "stream_capture");
+}

@@ -9,6 +9,7 @@ run time. There is no fallback: without the library every op raises.
 import ctypes
 import itertools
 import os
+import threading
 
 import torch  # noqa: F401  (loads the HIP runtime the library then shares)
 
@@ -100,6 +101,7 @@ SIGNATURES = {
     "qlx_quantize_act_int8": ([_P, _P, _P, _P, _P, _I, _I, _P], _I),
     "qlx_plan_linear": ([_I, _I, _I, _I, _I, _PLAN], _I),
     "qlx_plan_tickets": ([_PLAN, _I, _I, _I, _I], _I),
+    "qlx_stream_capture": ([_P, ctypes.POINTER(ctypes.c_ulonglong)], _I),
     "qlx_plan_fit": ([_PLAN, _I, _I, _I, _I, _I, _I], _I),
     "qlx_tile_rows": ([_P, _P, _I, _I, _P], _I),
     "qlx_linear_w8a16": ([_P, _P, _P, _P, _I, _I, _I, _I, _PLAN, _P], _I),
@@ -222,15 +224,49 @@ STREAM_SLOTS = 64
 _stream_tickets = {}
 
 
+class _Local(threading.local):
+    """The capture that this thread last launched into and its counters by stream."""
+
+    def __init__(self):
+        self.id = ctypes.c_ulonglong()
+        self.capture, self.counters = 0, {}
+
+
+_local = _Local()
+
+
+def capture_id(stream):
+    """The graph capture that ``stream`` (a handle) is in, 0 outside one."""
+    call("qlx_stream_capture", stream, _local.id)
+    return _local.id.value
+
+
+def _capture_tickets(device, stream, capture, count):
+    """``count`` counters for captured calls on ``stream`` (the current one). A graph's replays may overlap
+    any other call, on whichever stream, so its counters are its own: memory of its pool, zeroed by a node
+    of it (1.5 us a replay), shared by the calls that the capture puts one after the other on one stream."""
+    if _local.capture != capture:
+        _local.capture, _local.counters = capture, {}
+    buf = _local.counters.get(stream)
+    if buf is None or buf.numel() < count:
+        buf = _local.counters[stream] = torch.zeros(count, dtype=torch.int32, device=device)
+    return buf
+
+
 def stream_tickets(device, stream):
-    """The address of ``STREAM_TICKETS`` zeroed counters for one stream's split-K calls: calls that
-    overlap on different streams count apart (from the 65th stream on, slots are shared in turn)."""
+    """The address of ``STREAM_TICKETS`` zeroed counters for the split-K calls of one stream, or of one
+    stream of a graph capture: calls that overlap count apart (from the 65th stream on, slots are shared
+    in turn)."""
+    capture = capture_id(stream)
+    if capture:
+        return _capture_tickets(device, stream, capture, STREAM_TICKETS).data_ptr()
+    if _local.counters:  # an ended capture's: back to its pool
+        _local.capture, _local.counters = 0, {}
     index = device.index if device.index is not None else torch.cuda.current_device()
     pool = _stream_tickets.get(index)
     if pool is None:
         buf = torch.zeros(STREAM_SLOTS * STREAM_TICKETS, dtype=torch.int32, device=device)
-        if not torch.cuda.is_current_stream_capturing():  # once: other streams' first calls find it zeroed
-            torch.cuda.current_stream(device).synchronize()
+        torch.cuda.current_stream(device).synchronize()  # once: other streams' first calls find it zeroed
         pool = _stream_tickets.setdefault(index, (buf, {}, itertools.count()))
     buf, slots, count = pool
     slot = slots.get(stream)

@@ -204,6 +204,57 @@ def test_calls_of_two_streams_count_apart():
             assert (bits16(y) == want[i]).all()
 
 
+def captured(fmt, xs, ps, splits):
+    """A graph, on torch's own capture stream, of sliced calls one after the other."""
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = [resident(fmt, x, p, splits) for x, p in zip(xs, ps)]
+    return graph, outs
+
+
+def test_replays_that_overlap_count_apart():
+    """Graphs captured on one stream, replayed on two while the same calls run eagerly on a third: every
+    result is that of the calls one after the other."""
+    fmt, m, n, k = "w8a16", 8, 2560, 9728
+    ps = [make(fmt, n, k, seed)[1] for seed in (71, 72, 73)]
+    xs = [acts(m, k, seed) for seed in (74, 75, 76)]
+    want = [bits16(resident(fmt, x, p, 4)) for x, p in zip(xs, ps)]
+    graphs = [captured(fmt, xs, ps, 4) for _ in range(2)]
+    streams = [torch.cuda.Stream(DEV) for _ in range(3)]
+    for _ in range(4):
+        for _, outs in graphs:
+            for y in outs:
+                y.zero_()
+        torch.cuda.synchronize()
+        eager = []
+        for _ in range(4):
+            for st, (graph, _) in zip(streams, graphs):
+                with torch.cuda.stream(st):
+                    graph.replay()
+            with torch.cuda.stream(streams[2]):
+                eager.append([resident(fmt, x, p, 4) for x, p in zip(xs, ps)])
+        torch.cuda.synchronize()
+        for outs in [g[1] for g in graphs] + eager:
+            for y, w in zip(outs, want):
+                assert (bits16(y) == w).all()
+
+
+def test_the_first_sliced_call_may_be_a_captured_one(monkeypatch):
+    """Eager calls before the graph's first replay, and after it, find their own counters zeroed."""
+    monkeypatch.setattr(_lib, "_stream_tickets", {})
+    fmt, m, n, k = "w4a16", 4, 2560, 9728
+    p, x = make(fmt, n, k, 81)[1], acts(m, k, 82)
+    graph, (out,) = captured(fmt, [x], [p], 3)
+    eager = bits16(resident(fmt, x, p, 3))
+    close(resident(fmt, x, p, 3), decode(fmt, x, p, False), False, "eager before the replay")
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (bits16(out) == eager).all() and (bits16(resident(fmt, x, p, 3)) == eager).all()
+    assert all(int(buf.abs().sum()) == 0 for buf, _, _ in _lib._stream_tickets.values())
+
+
 @pytest.mark.parametrize("fmt,k,splits", [("w4a16", 8448, 4), ("fp8", 3328, 6), ("int4g64", 8448, 4)])
 def test_a_short_last_slice_of_one_token(fmt, k, splits):
     """A last K slice whose waves hold several units fewer than the others', the last of them at the end

@@ -1,9 +1,11 @@
 """The host side of the resident-activation GEMM (qlx_linear_resident): its plan on both sides of the
-kernel's size limits. Nothing here reaches a GPU."""
+kernel's size limits, and the counters of its K slices. Nothing here reaches a GPU."""
 
 import ctypes
+import types
 
 import pytest
+import torch
 
 from kernels import _lib
 
@@ -36,3 +38,44 @@ def test_plan_takes_no_call_that_the_kernel_refuses(name):
                 assert rc == _lib.QLX_EINVAL and "16-byte boundaries" in _lib.last_error(), (name, m, n, k, _lib.last_error())
                 assert n < edge, (name, m, n, k)
     assert served or name == "fp8"  # FP8 weights of over 64 MiB are left to another kernel
+
+
+@pytest.fixture
+def counters(monkeypatch):
+    """stream_tickets on CPU memory, its state put back afterwards; returns the capture of each stream."""
+    captures = {}
+    monkeypatch.setattr(_lib, "capture_id", lambda stream: captures.get(stream, 0), raising=False)
+    monkeypatch.setattr(_lib, "_stream_tickets", {})
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: types.SimpleNamespace(synchronize=lambda: None))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: bool(captures))
+    return captures
+
+
+def test_captured_calls_count_apart_from_every_other_call(counters):
+    """A graph's replays may overlap eager calls and other graphs' replays, whatever stream each was
+    captured on: one capture's calls on one stream share counters, no other calls do."""
+    cpu = torch.device("cpu", 0)
+    eager = _lib.stream_tickets(cpu, 16)
+    seen = {eager}
+    for capture in (1, 2):
+        counters.update({16: capture, 32: capture})  # the same streams captured again, one forked to
+        held = [_lib.stream_tickets(cpu, s) for s in (16, 32)]
+        keep = list(_lib._local.counters.values())  # the graph's memory
+        assert held == [_lib.stream_tickets(cpu, s) for s in (16, 32)]
+        assert len(seen | set(held)) == len(seen) + 2
+        seen |= set(held)
+        counters.clear()
+        assert _lib.stream_tickets(cpu, 16) == eager and not _lib._local.counters
+        assert all(int(buf.abs().sum()) == 0 for buf in keep)
+
+
+def test_a_capture_makes_no_counters_for_eager_calls(counters):
+    """The first sliced call of a device may be a captured one; the eager calls' counters are made, and
+    zeroed, by an eager call."""
+    cpu = torch.device("cpu", 0)
+    counters[16] = 7
+    _lib.stream_tickets(cpu, 16)
+    assert not _lib._stream_tickets
+    counters.clear()
+    _lib.stream_tickets(cpu, 16)
+    assert len(_lib._stream_tickets) == 1
