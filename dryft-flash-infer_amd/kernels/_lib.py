@@ -218,18 +218,20 @@ def tickets(device, count):
     return buf
 
 
-#: Counters of one stream's slot and slots of a device (64 x 2 KB).
+#: Counters of one stream's slot, and slots of a device (64 x 2 KB; torch's own pool has 32 streams). A slot
+#: stays its stream's; calls on streams past the 64th zero counters of their own.
 STREAM_TICKETS = 512
 STREAM_SLOTS = 64
 _stream_tickets = {}
 
 
 class _Local(threading.local):
-    """The capture that this thread last launched into and its counters by stream."""
+    """The capture that this thread last launched into, its counters by stream, and the counters of this
+    thread's last call without a slot (memory of that call's stream, so free for reuse once it is enqueued)."""
 
     def __init__(self):
         self.id = ctypes.c_ulonglong()
-        self.capture, self.counters = 0, {}
+        self.capture, self.counters, self.spare = 0, {}, None
 
 
 _local = _Local()
@@ -254,9 +256,8 @@ def _capture_tickets(device, stream, capture, count):
 
 
 def stream_tickets(device, stream):
-    """The address of ``STREAM_TICKETS`` zeroed counters for the split-K calls of one stream, or of one
-    stream of a graph capture: calls that overlap count apart (from the 65th stream on, slots are shared
-    in turn)."""
+    """The address of ``STREAM_TICKETS`` zeroed counters for the next split-K call on ``stream``: calls that
+    overlap count apart, whether on two streams, in two graphs or in one graph's branches."""
     capture = capture_id(stream)
     if capture:
         return _capture_tickets(device, stream, capture, STREAM_TICKETS).data_ptr()
@@ -270,6 +271,9 @@ def stream_tickets(device, stream):
         pool = _stream_tickets.setdefault(index, (buf, {}, itertools.count()))
     buf, slots, count = pool
     slot = slots.get(stream)
-    if slot is None:
-        slot = slots.setdefault(stream, next(count) % STREAM_SLOTS)
+    if slot is None and len(slots) < STREAM_SLOTS:
+        slot = slots.setdefault(stream, next(count))
+    if slot is None or slot >= STREAM_SLOTS:
+        _local.spare = torch.zeros(STREAM_TICKETS, dtype=torch.int32, device=device)
+        return _local.spare.data_ptr()
     return buf.data_ptr() + slot * STREAM_TICKETS * 4

@@ -79,3 +79,16 @@ def test_a_capture_makes_no_counters_for_eager_calls(counters):
     counters.clear()
     _lib.stream_tickets(cpu, 16)
     assert len(_lib._stream_tickets) == 1
+
+
+def test_streams_past_the_slots_share_none(counters):
+    """Each stream counts apart from the 64 that hold a slot, and from its neighbours, also past them."""
+    cpu = torch.device("cpu", 0)
+    at = [_lib.stream_tickets(cpu, 16 * s) for s in range(1, _lib.STREAM_SLOTS + 9)]
+    base = _lib._stream_tickets[0][0].data_ptr()
+    size = 4 * _lib.STREAM_TICKETS
+    assert sorted(at[:_lib.STREAM_SLOTS]) == [base + size * i for i in range(_lib.STREAM_SLOTS)]
+    assert all(not base <= a < base + size * _lib.STREAM_SLOTS for a in at[_lib.STREAM_SLOTS:])
+    assert all(a != b for a, b in zip(at[_lib.STREAM_SLOTS:], at[_lib.STREAM_SLOTS + 1:]))
+    assert len(_lib._stream_tickets[0][1]) == _lib.STREAM_SLOTS
+    assert at[:_lib.STREAM_SLOTS] == [_lib.stream_tickets(cpu, 16 * s) for s in range(1, _lib.STREAM_SLOTS + 1)]
