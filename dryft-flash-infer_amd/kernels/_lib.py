@@ -203,26 +203,12 @@ def require_device(*tensors):
             raise ValueError("tensors must be contiguous")
 
 
-_tickets = {}
-
-
-def tickets(device, count):
-    """Per-device ticket counters for split-K, zero between calls (kernels reset them)."""
-    index = device.index if isinstance(device, torch.device) else torch.device(device).index
-    index = index or 0
-    buf = _tickets.get(index)
-    if buf is None or buf.numel() < count:
-        size = max(count, 1 << 16)
-        buf = torch.zeros(size, dtype=torch.int32, device=device)
-        _tickets[index] = buf
-    return buf
-
-
 #: Counters of one stream's slot, and slots of a device (64 x 2 KB; torch's own pool has 32 streams). A slot
 #: stays its stream's; calls on streams past the 64th zero counters of their own.
 STREAM_TICKETS = 512
 STREAM_SLOTS = 64
 _stream_tickets = {}
+_tickets = {}
 
 
 class _Local(threading.local):
@@ -277,3 +263,19 @@ def stream_tickets(device, stream):
         _local.spare = torch.zeros(STREAM_TICKETS, dtype=torch.int32, device=device)
         return _local.spare.data_ptr()
     return buf.data_ptr() + slot * STREAM_TICKETS * 4
+
+
+def tickets(device, count):
+    """``count`` zeroed counters for the next split-K call on ``device``'s current stream, apart from every
+    call that may overlap it as in ``stream_tickets``; the caller holds the tensor until it has launched."""
+    st = stream(device)
+    capture = capture_id(st)
+    if capture:
+        return _capture_tickets(device, st, capture, max(count, STREAM_TICKETS))
+    key = (device.index if device.index is not None else torch.cuda.current_device(), st)
+    buf = _tickets.get(key)
+    if buf is None or buf.numel() < count:
+        buf = torch.zeros(max(count, 1 << 12), dtype=torch.int32, device=device)
+        if key in _tickets or len(_tickets) < STREAM_SLOTS:
+            _tickets[key] = buf
+    return buf

@@ -7,6 +7,8 @@ outputs within one bf16 rounding step: 2^-7 of the value plus 2^-9 of the row's 
 roundings more, 2^-6), and the oracle's dequantize-then-matmul at a rel-L2 of 1e-2. A
 zero weight row gives exactly zero; fp32 planes summed in slice order are the reduced output."""
 
+import functools
+
 import numpy as np
 import pytest
 import torch
@@ -204,22 +206,30 @@ def test_calls_of_two_streams_count_apart():
             assert (bits16(y) == want[i]).all()
 
 
-def captured(fmt, xs, ps, splits):
-    """A graph, on torch's own capture stream, of sliced calls one after the other."""
+def sliced(kernel, x, p):
+    """A W8A16 call in K slices on one kernel."""
+    if kernel == "resident":
+        return resident("w8a16", x, p, 4)
+    return qlinear.linear_w8a16(x, p.tiles, skinny=True) if kernel == "skinny" else \
+        qlinear.linear_w8a16(x, p.tiles, config=(8, 8, 1, 4))
+
+
+def captured(calls):
+    """A graph of calls one after the other, on torch's own capture stream."""
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        outs = [resident(fmt, x, p, splits) for x, p in zip(xs, ps)]
+        outs = [fn() for fn in calls]
     return graph, outs
 
 
-def test_replays_that_overlap_count_apart():
+@pytest.mark.parametrize("kernel", ["resident", "skinny", "decode"])
+def test_replays_that_overlap_count_apart(kernel):
     """Graphs captured on one stream, replayed on two while the same calls run eagerly on a third: every
     result is that of the calls one after the other."""
-    fmt, m, n, k = "w8a16", 8, 2560, 9728
-    ps = [make(fmt, n, k, seed)[1] for seed in (71, 72, 73)]
-    xs = [acts(m, k, seed) for seed in (74, 75, 76)]
-    want = [bits16(resident(fmt, x, p, 4)) for x, p in zip(xs, ps)]
-    graphs = [captured(fmt, xs, ps, 4) for _ in range(2)]
+    m, n, k = 8, 2560, 9728
+    calls = [functools.partial(sliced, kernel, acts(m, k, seed + 3), make("w8a16", n, k, seed)[1]) for seed in (71, 72, 73)]
+    want = [bits16(fn()) for fn in calls]
+    graphs = [captured(calls) for _ in range(2)]
     streams = [torch.cuda.Stream(DEV) for _ in range(3)]
     for _ in range(4):
         for _, outs in graphs:
@@ -232,7 +242,7 @@ def test_replays_that_overlap_count_apart():
                 with torch.cuda.stream(st):
                     graph.replay()
             with torch.cuda.stream(streams[2]):
-                eager.append([resident(fmt, x, p, 4) for x, p in zip(xs, ps)])
+                eager.append([fn() for fn in calls])
         torch.cuda.synchronize()
         for outs in [g[1] for g in graphs] + eager:
             for y, w in zip(outs, want):
@@ -244,7 +254,7 @@ def test_the_first_sliced_call_may_be_a_captured_one(monkeypatch):
     monkeypatch.setattr(_lib, "_stream_tickets", {})
     fmt, m, n, k = "w4a16", 4, 2560, 9728
     p, x = make(fmt, n, k, 81)[1], acts(m, k, 82)
-    graph, (out,) = captured(fmt, [x], [p], 3)
+    graph, (out,) = captured([lambda: resident(fmt, x, p, 3)])
     eager = bits16(resident(fmt, x, p, 3))
     close(resident(fmt, x, p, 3), decode(fmt, x, p, False), False, "eager before the replay")
     for _ in range(3):

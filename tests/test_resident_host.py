@@ -1,5 +1,5 @@
 """The host side of the resident-activation GEMM (qlx_linear_resident): its plan on both sides of the
-kernel's size limits, and the counters of its K slices. Nothing here reaches a GPU."""
+kernel's size limits; and the counters of its and the other kernels' K slices. Nothing here reaches a GPU."""
 
 import ctypes
 import types
@@ -42,10 +42,11 @@ def test_plan_takes_no_call_that_the_kernel_refuses(name):
 
 @pytest.fixture
 def counters(monkeypatch):
-    """stream_tickets on CPU memory, its state put back afterwards; returns the capture of each stream."""
+    """The counters on CPU memory, their state put back afterwards; returns the capture of each stream."""
     captures = {}
     monkeypatch.setattr(_lib, "capture_id", lambda stream: captures.get(stream, 0), raising=False)
     monkeypatch.setattr(_lib, "_stream_tickets", {})
+    monkeypatch.setattr(_lib, "_tickets", {})
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device: types.SimpleNamespace(synchronize=lambda: None))
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: bool(captures))
     return captures
@@ -92,3 +93,23 @@ def test_streams_past_the_slots_share_none(counters):
     assert all(a != b for a, b in zip(at[_lib.STREAM_SLOTS:], at[_lib.STREAM_SLOTS + 1:]))
     assert len(_lib._stream_tickets[0][1]) == _lib.STREAM_SLOTS
     assert at[:_lib.STREAM_SLOTS] == [_lib.stream_tickets(cpu, 16 * s) for s in range(1, _lib.STREAM_SLOTS + 1)]
+
+
+def test_the_other_kernels_calls_count_apart_too(counters, monkeypatch):
+    """tickets() of the decode and skinny kernels: by stream, a capture's own, more of them when asked."""
+    cpu = torch.device("cpu", 0)
+
+    def at(stream, count=160):
+        monkeypatch.setattr(_lib, "stream", lambda device: stream)
+        buf = _lib.tickets(cpu, count)
+        assert buf.numel() >= count and not buf.any()
+        return buf
+
+    eager = [at(16 * s) for s in range(1, _lib.STREAM_SLOTS + 4)]
+    assert len({b.data_ptr() for b in eager}) == len(eager) and len(_lib._tickets) == _lib.STREAM_SLOTS
+    assert at(16) is eager[0] and at(16, 9496) is at(16, 9496) is not eager[0]
+    counters.update({16: 3, 32: 3})
+    held = [at(16), at(32), at(16)]
+    assert held[0] is held[2] is not held[1] and all(b is not h for b in _lib._tickets.values() for h in held)
+    counters.update({16: 4})
+    assert at(16) is not held[0]
