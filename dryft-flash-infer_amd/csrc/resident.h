@@ -35,6 +35,7 @@ struct ResidentArgs {
   const void* x;
   const float* xs;  // FP8: token scales
   uint16_t* y;
+  float* sum;  // the fp32 output of QLX_MODE_SUM in several slices
   float* work;
   int* tickets;
   int m, n, k, half, swiglu;
@@ -499,6 +500,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) r
       const size_t o = (size_t)(m0 + mm) * a.half + row;
       store_pair(a.y, o, swiglu_bf(gv[0], uv[0]), swiglu_bf(gv[1], uv[1]));
       store_pair(a.y, o + 2, swiglu_bf(gv[2], uv[2]), swiglu_bf(gv[3], uv[3]));
+    } else if (a.sum) {
+      *gmem(reinterpret_cast<f32x4*>(a.sum + (size_t)(m0 + mm) * a.n + row)) = gv;
     } else {
       const size_t o = (size_t)(m0 + mm) * a.n + row;
       store_pair(a.y, o, gv[0], gv[1]);
@@ -591,7 +594,7 @@ int resident_run(const char* name, ResidentArgs a, int m, int n, int k, const ql
   QLX_REQUIRE(m >= 1 && m <= 64, "%s: m=%d must be in 1..64", name, m);
   QLX_REQUIRE(n >= 16 && n % 16 == 0 && k >= 128 && k % 128 == 0 && k % F::KSTEP == 0,
               "%s: n=%d k=%d do not fit the tiled format", name, n, k);
-  QLX_REQUIRE(plan->mode >= QLX_MODE_BF16 && plan->mode <= QLX_MODE_SWIGLU, "%s: mode %d", name, plan->mode);
+  QLX_REQUIRE(plan->mode >= QLX_MODE_BF16 && plan->mode <= QLX_MODE_SUM, "%s: mode %d", name, plan->mode);
   const int units = k / Unit<F>::KV;
   QLX_REQUIRE(plan->splits >= 1 && plan->splits <= units, "%s: splits must be 1..%d", name, units);
   ResidentPlan p;
@@ -602,7 +605,8 @@ int resident_run(const char* name, ResidentArgs a, int m, int n, int k, const ql
   // 16-byte buffer loads of weights and activations, 4-byte ones of scales
   QLX_REQUIRE(((uintptr_t)a.w | (uintptr_t)a.x) % 16 == 0 && ((uintptr_t)a.ws | (uintptr_t)a.y) % 4 == 0,
               "%s: operands must start on 16-byte boundaries (scales, outputs: 4)", name);
-  const bool planes = plan->mode == QLX_MODE_PLANES;
+  QLX_REQUIRE(plan->mode != QLX_MODE_SUM || (uintptr_t)a.y % 16 == 0, "%s: fp32 outputs must start on a 16-byte boundary", name);
+  const bool planes = plan->mode == QLX_MODE_PLANES, sum = plan->mode == QLX_MODE_SUM;
   QLX_REQUIRE(!planes || p.splits == plan->splits, "%s: %d splits leave %d non-empty planes", name, plan->splits, p.splits);
   QLX_REQUIRE(planes ? plan->workspace != nullptr
                      : p.splits == 1 || (plan->workspace != nullptr && plan->tickets != nullptr),
@@ -614,8 +618,9 @@ int resident_run(const char* name, ResidentArgs a, int m, int n, int k, const ql
   a.strided = p.splits == 1 && a.run >= 12;
   a.wbytes = (unsigned)((long long)(n / 16) * units * 1024);
   a.sbytes = (unsigned)((long long)n * (Unit<F>::NG ? units * Unit<F>::NG : 1) * 2);
-  a.planes = planes || p.splits > 1;
-  a.work = plan->workspace, a.tickets = !planes && p.splits > 1 ? plan->tickets : nullptr;
+  a.planes = planes || sum || p.splits > 1;
+  a.sum = sum ? reinterpret_cast<float*>(a.y) : nullptr;
+  a.work = sum && p.splits == 1 ? a.sum : plan->workspace, a.tickets = !planes && p.splits > 1 ? plan->tickets : nullptr;
   const hipError_t e = m <= 16 ? resident_units<F, 1>(a, p.u, (hipStream_t)stream)
                                : resident_units<F, 2>(a, p.u, (hipStream_t)stream);
   return hip_status(e, name);

@@ -64,7 +64,7 @@ extern "C" {
 int qlx_plan_resident(int fmt, int mode, int m, int n, int k, qlx_plan* plan) {
   QLX_REQUIRE(plan != nullptr, "plan is NULL");
   const int kstep = fmt == QLX_FMT_W4A16 ? 256 : 128;
-  QLX_REQUIRE(mode >= QLX_MODE_BF16 && mode <= QLX_MODE_SWIGLU, "bad mode %d", mode);
+  QLX_REQUIRE(mode >= QLX_MODE_BF16 && mode <= QLX_MODE_SUM, "bad mode %d", mode);
   QLX_REQUIRE(m >= 1 && m <= 64 && n >= 16 && n % 16 == 0 && k >= kstep && k % kstep == 0,
               "shape m=%d n=%d k=%d does not fit format %d", m, n, k, fmt);
   const int s = resident_splits_of(fmt, m, n, k);

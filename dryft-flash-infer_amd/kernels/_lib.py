@@ -17,7 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libqlinear.so")
 
 QLX_OK, QLX_EINVAL, QLX_EHIP = 0, -1, -2
-MODE_BF16, MODE_PLANES, MODE_SWIGLU = 0, 1, 2
+MODE_BF16, MODE_PLANES, MODE_SWIGLU, MODE_SUM = 0, 1, 2, 3
 SCALE_F16, SCALE_BF16 = 0, 1
 STORE_OFFSET, STORE_SIGNED, STORE_K32 = 0, 1, 2
 FMT_W8A16, FMT_W4A16, FMT_FP8, FMT_REF8, FMT_REF4, FMT_FP8WO, FMT_INT8 = range(7)

@@ -250,23 +250,22 @@ def _fmt(prepared):
 def _resident_plan(prepared, batch, config, mode):
     """The resident GEMM's plan (``qlx_linear_resident``) for a call on tiled reference-format weights,
     or None: a config that asks for K slices gets them from the decode kernel, whose planes sum to
-    its result. A config of one slice leaves the slices to the library: where the decode kernel
-    would cut K to fit its LDS, the planes are the resident GEMM's too."""
+    its result. A config of one slice leaves the slices to the library, and its planes come from the
+    resident GEMM as ``matmul``'s result does: the slices themselves where the decode kernel would cut
+    K to fit its LDS, else one plane, their sum."""
     if prepared.fmt != "ref" or not prepared.tiled or batch > 64:
         return None
     if mode != _lib.MODE_SWIGLU and _splitk(prepared, config) > 1:
         return None
     fmt = _fmt(prepared)
-    if mode == _lib.MODE_PLANES:
-        cfg = _plan_config(prepared, batch, config, mode)
-        if _linear.splits_for(fmt, mode, batch, prepared.rows, prepared.k, cfg, fit=True) == 1:
-            return None
     from . import qlinear
     if not qlinear.aligned(prepared.weight, prepared.scale):
         return None
     plan = qlinear.plan_resident(fmt, batch, prepared.rows, prepared.k, mode == _lib.MODE_SWIGLU)
-    if plan is not None:
-        plan.mode = mode
+    if plan is not None and mode == _lib.MODE_PLANES:
+        cfg = _plan_config(prepared, batch, config, mode)
+        one = _linear.splits_for(fmt, mode, batch, prepared.rows, prepared.k, cfg, fit=True) == 1
+        plan.mode = _lib.MODE_SUM if one else mode
     return plan
 
 
@@ -298,7 +297,7 @@ def splits(prepared: Prepared, batch: int, config=(4, 1)) -> int:
     """How many fp32 planes ``matmul_partials`` returns for this shape and config."""
     plan = _resident_plan(prepared, batch, config, _lib.MODE_PLANES)
     if plan is not None:
-        return plan.splits
+        return 1 if plan.mode == _lib.MODE_SUM else plan.splits
     cfg = _plan_config(prepared, batch, config, _lib.MODE_PLANES)
     return _linear.splits_for(_fmt(prepared), _lib.MODE_PLANES, batch, prepared.rows, prepared.k, cfg, fit=True)
 

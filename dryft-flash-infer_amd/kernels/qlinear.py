@@ -212,8 +212,8 @@ def plan_resident(fmt, m, n, k, swiglu=False):
 
 
 def run_resident(plan, fmt, q, s, x, xs, m, n, k):
-    """``qlx_linear_resident`` with ``plan``: bf16 ``[m, n]`` (SwiGLU ``[m, n/2]``), or fp32 planes
-    ``[splits, m, n]`` where the plan's mode is planes."""
+    """``qlx_linear_resident`` with ``plan``: bf16 ``[m, n]`` (SwiGLU ``[m, n/2]``); where the plan's mode is
+    planes, fp32 ``[splits, m, n]``, where it is their sum, ``[1, m, n]``."""
     device = x.device
     stream = _lib.stream(device)
     planes = plan.mode == _lib.MODE_PLANES
@@ -224,7 +224,10 @@ def run_resident(plan, fmt, q, s, x, xs, m, n, k):
         work = torch.empty((plan.splits, m, n), dtype=torch.float32, device=device)
         plan.workspace = work.data_ptr()
     if not planes:
-        out = torch.empty((m, n // 2 if plan.mode == _lib.MODE_SWIGLU else n), dtype=torch.bfloat16, device=device)
+        if plan.mode == _lib.MODE_SUM:
+            out = torch.empty((1, m, n), dtype=torch.float32, device=device)
+        else:
+            out = torch.empty((m, n // 2 if plan.mode == _lib.MODE_SWIGLU else n), dtype=torch.bfloat16, device=device)
         if plan.splits > 1:
             plan.tickets = _lib.stream_tickets(device, stream)
     _lib.call("qlx_linear_resident", fmt, _lib.ptr(q), _lib.ptr(s), _lib.ptr(x), _lib.ptr(xs), _lib.ptr(out), m, n, k,

@@ -44,6 +44,7 @@ extern "C" {
 /* linear modes */
 #define QLX_MODE_BF16 0   /* y[m][n] bf16 */
 #define QLX_MODE_PLANES 1 /* fp32 split-K planes [splits][m][n], not reduced */
+#define QLX_MODE_SUM 3    /* fp32 y [m][n], the K slices summed in slice order (qlx_linear_resident only) */
 #define QLX_MODE_SWIGLU 2 /* weight rows = [gate; up] (2I), y[m][i] = bf16(bf16(silu(g)) * u) */
 
 /* Launch plan of a linear call. `splits` K-slices run as separate workgroups; with
@@ -186,8 +187,8 @@ int qlx_linear_skinny_fp8(const void* w, const void* w_scale, const void* x_code
  * FP8, and the reference's tiled REF8 / REF4): each wave keeps its K range's activation fragments
  * in registers for the whole launch and streams that range of a run of 16-row weight tiles. FP8
  * takes the activation quantized beforehand (e4m3 codes, x_scale fp32 [m]); the others bf16 x and
- * no x_scale. Output bf16, SwiGLU, or the fp32 planes themselves (QLX_MODE_PLANES, in plan->workspace,
- * y unused); weights and planes of under 2 GiB each; w and x on 16-byte boundaries. qlx_plan_resident
+ * no x_scale. Output bf16, SwiGLU, their fp32 sum (QLX_MODE_SUM: rounded, the bf16 output's bits), or the
+ * fp32 planes themselves (QLX_MODE_PLANES, in plan->workspace, y unused); weights and planes of under 2 GiB each; w and x on 16-byte boundaries. qlx_plan_resident
  * fills plan->splits: 0 where no slice count fits the registers and those sizes, or another kernel
  * measured faster (qlx_linear_* / qlx_linear_skinny* serve those calls). With splits > 1 the call takes a workspace
  * of splits * m * n floats and 512 zeroed tickets (zero again afterwards). */

@@ -50,12 +50,12 @@ def decode(fmt, x, p, swiglu):
     return qlinear.FORMATS[fmt][1](x, p.tiles, config=cfg, swiglu=swiglu)
 
 
-def resident(fmt, x, p, splits, swiglu=False, planes=False):
+def resident(fmt, x, p, splits, swiglu=False, planes=False, mode=None):
     xs = None
     if fmt == "fp8":
         x, xs = qlinear.quantize_fp8_activation(x)
     plan = _lib.Plan()
-    plan.mode = _lib.MODE_PLANES if planes else (_lib.MODE_SWIGLU if swiglu else _lib.MODE_BF16)
+    plan.mode = mode or (_lib.MODE_PLANES if planes else (_lib.MODE_SWIGLU if swiglu else _lib.MODE_BF16))
     plan.splits = splits
     return qlinear.run_resident(plan, FMTS[fmt], p.weight, p.scale, x, xs, x.shape[0], p.rows, p.k)
 
@@ -98,7 +98,7 @@ def test_resident_planes_and_oracle(fmt):
     for m in (3, 24, 64):
         print(f"resident planes {fmt} m={m}", flush=True)
         x = acts(m, k, m)
-        for s in (2, 4):
+        for s in (1, 2, 4):
             got = resident(fmt, x, p, s)
             planes = resident(fmt, x, p, s, planes=True)
             acc = torch.zeros_like(planes[0])
@@ -108,6 +108,8 @@ def test_resident_planes_and_oracle(fmt):
                 assert ((acc - got.float()).abs() <= 2.0 ** -8 * got.float().abs() + 1e-6).all()
             else:
                 assert torch.equal(acc.to(torch.bfloat16), got), (fmt, m, s)
+            one = resident(fmt, x, p, s, mode=_lib.MODE_SUM)
+            assert one.shape == (1, m, n) and torch.equal(one[0], acc) and torch.equal(one[0].to(torch.bfloat16), got), (fmt, m, s)
         if fmt == "fp8":
             want = O.linear_fp8_w8a8(bits16(x), packed[0].view(torch.uint8).cpu().numpy(), bits16(packed[1])[:, None])
         else:
@@ -152,7 +154,7 @@ def test_operands_off_a_16_byte_boundary():
 
 def test_reference_format_planes_count():
     """cuda_fp8.splits names the planes matmul_partials returns, whichever kernel makes them; their
-    sum is matmul's result where there are several."""
+    sum is matmul's result."""
     for fmt in ("int8g64", "int4g64"):
         _, p = make(fmt, 2560, 9728, 6)
         for m in (1, 8, 33, 64):
@@ -160,11 +162,10 @@ def test_reference_format_planes_count():
                 x = acts(m, 9728, m)
                 planes = cuda_fp8.matmul_partials(x, p, config)
                 assert planes.shape[0] == cuda_fp8.splits(p, m, config), (fmt, m, config)
-                if planes.shape[0] > 1:
-                    acc = torch.zeros_like(planes[0])
-                    for plane in planes:
-                        acc += plane
-                    assert torch.equal(acc.to(torch.bfloat16), cuda_fp8.matmul(x, p, config)), (fmt, m, config)
+                acc = torch.zeros_like(planes[0])
+                for plane in planes:
+                    acc += plane
+                assert torch.equal(acc.to(torch.bfloat16), cuda_fp8.matmul(x, p, config)), (fmt, m, config)
 
 
 def test_graph_replays_equal_eager():
