@@ -160,12 +160,11 @@ extern "C" int qlx_plan_fit(qlx_plan* plan, int fmt, int m, int n, int k, int co
 }
 
 // The capture that a stream is in (0: none), the same for every stream that the capture has forked to.
-extern "C" int qlx_stream_capture(void* stream, unsigned long long* id) {
-  QLX_REQUIRE(id != nullptr, "stream_capture: id is NULL");
-  *id = 0;
-  if (stream == nullptr) return QLX_OK;  // the default stream cannot be captured
+// A stream that the runtime refuses to query counts as not captured: the launch on it reports the error.
+extern "C" unsigned long long qlx_stream_capture(void* stream) {
+  if (stream == nullptr) return 0;  // the default stream cannot be captured
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  const hipError_t e = hipStreamGetCaptureInfo((hipStream_t)stream, &status, id);
-  if (status == hipStreamCaptureStatusNone) *id = 0;
-  return qlx::hip_status(e, "stream_capture");
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo((hipStream_t)stream, &status, &id) != hipSuccess) return 0;
+  return status == hipStreamCaptureStatusNone ? 0 : id;
 }

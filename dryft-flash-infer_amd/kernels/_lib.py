@@ -101,7 +101,7 @@ SIGNATURES = {
     "qlx_quantize_act_int8": ([_P, _P, _P, _P, _P, _I, _I, _P], _I),
     "qlx_plan_linear": ([_I, _I, _I, _I, _I, _PLAN], _I),
     "qlx_plan_tickets": ([_PLAN, _I, _I, _I, _I], _I),
-    "qlx_stream_capture": ([_P, ctypes.POINTER(ctypes.c_ulonglong)], _I),
+    "qlx_stream_capture": ([_P], ctypes.c_ulonglong),
     "qlx_plan_fit": ([_PLAN, _I, _I, _I, _I, _I, _I], _I),
     "qlx_tile_rows": ([_P, _P, _I, _I, _P], _I),
     "qlx_linear_w8a16": ([_P, _P, _P, _P, _I, _I, _I, _I, _PLAN, _P], _I),
@@ -216,7 +216,6 @@ class _Local(threading.local):
     thread's last call without a slot (memory of that call's stream, so free for reuse once it is enqueued)."""
 
     def __init__(self):
-        self.id = ctypes.c_ulonglong()
         self.capture, self.counters, self.spare = 0, {}, None
 
 
@@ -225,8 +224,7 @@ _local = _Local()
 
 def capture_id(stream):
     """The graph capture that ``stream`` (a handle) is in, 0 outside one."""
-    call("qlx_stream_capture", stream, _local.id)
-    return _local.id.value
+    return lib().qlx_stream_capture(stream)
 
 
 def _capture_tickets(device, stream, capture, count):

@@ -140,7 +140,7 @@ int qlx_plan_linear(int fmt, int mode, int m, int n, int k, qlx_plan* plan);
 int qlx_plan_tickets(const qlx_plan* plan, int fmt, int m, int n, int k);
 /* The id of the graph capture that `stream` is in, 0 outside one: a captured call's tickets have to be
  * the graph's own, zeroed in it, as its replays may overlap any other call. */
-int qlx_stream_capture(void* stream, unsigned long long* id);
+unsigned long long qlx_stream_capture(void* stream);
 /* Normalise plan->splits so every K slice is non-empty; with `grow`, first raise it until the
  * plan's LDS fits (the reference's _plan, engine/kernels/cuda_fp8.py:1255-1276). comp =
  * activation components (2 only for QLX_FMT_INT8 with a residual component). */
