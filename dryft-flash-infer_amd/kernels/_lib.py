@@ -203,20 +203,21 @@ def require_device(*tensors):
             raise ValueError("tensors must be contiguous")
 
 
-#: Counters of one stream's slot, and slots of a device (64 x 2 KB; torch's own pool has 32 streams). A slot
-#: stays its stream's; calls on streams past the 64th zero counters of their own.
+#: Counters of a slot and slots of a device (256 x 2 KB). A slot stays with its stream, or with its stream of
+#: one graph capture, whose graph may be replayed at any later time; calls past the last slot, and those
+#: that need more counters, zero their own.
 STREAM_TICKETS = 512
-STREAM_SLOTS = 64
+STREAM_SLOTS = 256
 _stream_tickets = {}
-_tickets = {}
 
 
 class _Local(threading.local):
-    """The capture that this thread last launched into, its counters by stream, and the counters of this
-    thread's last call without a slot (memory of that call's stream, so free for reuse once it is enqueued)."""
+    """The capture that this thread last launched into (0: none), and its counters outside the slots by
+    device and stream. A buffer is memory of its stream, so it may go once the call is enqueued; a
+    capture's is memory of its graph."""
 
     def __init__(self):
-        self.capture, self.counters, self.spare = 0, {}, None
+        self.capture, self.counters = 0, {}
 
 
 _local = _Local()
@@ -227,53 +228,35 @@ def capture_id(stream):
     return lib().qlx_stream_capture(stream)
 
 
-def _capture_tickets(device, stream, capture, count):
-    """``count`` counters for captured calls on ``stream`` (the current one). A graph's replays may overlap
-    any other call, on whichever stream, so its counters are its own: memory of its pool, zeroed by a node
-    of it (1.5 us a replay), shared by the calls that the capture puts one after the other on one stream."""
-    if _local.capture != capture:
-        _local.capture, _local.counters = capture, {}
-    buf = _local.counters.get(stream)
-    if buf is None or buf.numel() < count:
-        buf = _local.counters[stream] = torch.zeros(count, dtype=torch.int32, device=device)
-    return buf
-
-
-def stream_tickets(device, stream):
-    """The address of ``STREAM_TICKETS`` zeroed counters for the next split-K call on ``stream``: calls that
-    overlap count apart, whether on two streams, in two graphs or in one graph's branches."""
+def stream_tickets(device, stream, count=STREAM_TICKETS):
+    """The address of ``count`` zeroed counters for this thread's next split-K call on ``stream``, the current
+    one: calls that may overlap count apart, whether on two streams, in two graphs' replays (whatever
+    stream they were captured on) or in one graph's branches. The slots are made by eager calls: inside a
+    capture their zeroing would be a node of that graph. Counters zeroed in a capture cost its replays
+    that node, 1 to 4 us."""
     capture = capture_id(stream)
-    if capture:
-        return _capture_tickets(device, stream, capture, STREAM_TICKETS).data_ptr()
-    if _local.counters:  # an ended capture's: back to its pool
-        _local.capture, _local.counters = 0, {}
     index = device.index if device.index is not None else torch.cuda.current_device()
     pool = _stream_tickets.get(index)
-    if pool is None:
+    if pool is None and not capture:
         buf = torch.zeros(STREAM_SLOTS * STREAM_TICKETS, dtype=torch.int32, device=device)
         torch.cuda.current_stream(device).synchronize()  # once: other streams' first calls find it zeroed
         pool = _stream_tickets.setdefault(index, (buf, {}, itertools.count()))
-    buf, slots, count = pool
-    slot = slots.get(stream)
-    if slot is None and len(slots) < STREAM_SLOTS:
-        slot = slots.setdefault(stream, next(count))
-    if slot is None or slot >= STREAM_SLOTS:
-        _local.spare = torch.zeros(STREAM_TICKETS, dtype=torch.int32, device=device)
-        return _local.spare.data_ptr()
-    return buf.data_ptr() + slot * STREAM_TICKETS * 4
+    if pool is not None and count <= STREAM_TICKETS:
+        buf, slots, numbers = pool
+        slot = slots.get((stream, capture))
+        if slot is None and len(slots) < STREAM_SLOTS:
+            slot = slots.setdefault((stream, capture), next(numbers))
+        if slot is not None and slot < STREAM_SLOTS:
+            return buf.data_ptr() + slot * STREAM_TICKETS * 4
+    if _local.capture != capture or len(_local.counters) > 64:
+        _local.capture, _local.counters = capture, {}
+    buf = _local.counters.get((index, stream))
+    if buf is None or buf.numel() < count:
+        buf = torch.zeros(max(count, STREAM_TICKETS), dtype=torch.int32, device=device)
+        _local.counters[index, stream] = buf
+    return buf.data_ptr()
 
 
 def tickets(device, count):
-    """``count`` zeroed counters for the next split-K call on ``device``'s current stream, apart from every
-    call that may overlap it as in ``stream_tickets``; the caller holds the tensor until it has launched."""
-    st = stream(device)
-    capture = capture_id(st)
-    if capture:
-        return _capture_tickets(device, st, capture, max(count, STREAM_TICKETS))
-    key = (device.index if device.index is not None else torch.cuda.current_device(), st)
-    buf = _tickets.get(key)
-    if buf is None or buf.numel() < count:
-        buf = torch.zeros(max(count, 1 << 12), dtype=torch.int32, device=device)
-        if key in _tickets or len(_tickets) < STREAM_SLOTS:
-            _tickets[key] = buf
-    return buf
+    """``stream_tickets`` for a call on ``device``'s current stream."""
+    return stream_tickets(device, stream(device), count)

@@ -48,8 +48,7 @@ def run(fmt, entry, x, n, k, args_before_y, args_after_dims=(), mode=_lib.MODE_B
             work = torch.empty((splits, m, n), dtype=torch.float32, device=device)
             plan.workspace = work.data_ptr()
             count = _lib.lib().qlx_plan_tickets(plan, fmt, m, n, k)
-            counters = _lib.tickets(device, count)
-            plan.tickets = counters.data_ptr()
+            plan.tickets = _lib.tickets(device, count)
     _lib.call(entry, *args_before_y, _lib.ptr(out), m, n, k, *args_after_dims,
               ctypes.byref(plan), _lib.stream(device))
     return out
@@ -70,8 +69,7 @@ def run_add_norm(fmt, weight_args, x, n, k, tiled, residual, norm_weight, eps, d
         work = torch.empty((plan.splits, m, n), dtype=torch.float32, device=device)
         plan.workspace = work.data_ptr()
         count = _lib.lib().qlx_plan_tickets(plan, fmt, m, n, k)
-        counters = _lib.tickets(device, count)
-        plan.tickets = counters.data_ptr()
+        plan.tickets = _lib.tickets(device, count)
     res = torch.empty_like(residual)
     normed = torch.empty_like(residual)
     w, ws = weight_args

@@ -190,8 +190,7 @@ def _skinny(fmt, q, s, x, n, k, swiglu, fused_reduce=None):
         work = torch.empty((plan.splits, m, n), dtype=torch.float32, device=x.device)
         plan.workspace = work.data_ptr()
         if fused_reduce:  # one counter per row group: n / 16 always suffices
-            counters = _lib.tickets(x.device, n // 16)
-            plan.tickets = counters.data_ptr()
+            plan.tickets = _lib.tickets(x.device, n // 16)
     _lib.call("qlx_linear_skinny", fmt, _lib.ptr(q), _lib.ptr(s), _lib.ptr(x), _lib.ptr(out), m, n, k,
               ctypes.byref(plan), _lib.stream(x.device))
     return out
@@ -318,8 +317,7 @@ def _skinny_fp8(q, s, xq, sx, n, k, swiglu, fused_reduce=None):
         work = torch.empty((plan.splits, m, n), dtype=torch.float32, device=xq.device)
         plan.workspace = work.data_ptr()
         if fused_reduce:
-            counters = _lib.tickets(xq.device, n // 16)
-            plan.tickets = counters.data_ptr()
+            plan.tickets = _lib.tickets(xq.device, n // 16)
     _lib.call("qlx_linear_skinny_fp8", _lib.ptr(q), _lib.ptr(s), _lib.ptr(xq), _lib.ptr(sx), _lib.ptr(out), m, n, k,
               ctypes.byref(plan), _lib.stream(xq.device))
     return out

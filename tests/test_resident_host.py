@@ -46,70 +46,83 @@ def counters(monkeypatch):
     captures = {}
     monkeypatch.setattr(_lib, "capture_id", lambda stream: captures.get(stream, 0), raising=False)
     monkeypatch.setattr(_lib, "_stream_tickets", {})
-    monkeypatch.setattr(_lib, "_tickets", {})
+    monkeypatch.setattr(_lib, "_local", _lib._Local())
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device: types.SimpleNamespace(synchronize=lambda: None))
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: bool(captures))
     return captures
+
+
+CPU = torch.device("cpu", 0)
+SIZE = 4 * _lib.STREAM_TICKETS
+
+
+def in_slots(address):
+    base = _lib._stream_tickets[0][0].data_ptr()
+    return base <= address < base + SIZE * _lib.STREAM_SLOTS
 
 
 def test_captured_calls_count_apart_from_every_other_call(counters):
     """A graph's replays may overlap eager calls and other graphs' replays, whatever stream each was
     captured on: one capture's calls on one stream share counters, no other calls do."""
-    cpu = torch.device("cpu", 0)
-    eager = _lib.stream_tickets(cpu, 16)
+    eager = _lib.stream_tickets(CPU, 16)
     seen = {eager}
-    for capture in (1, 2):
+    for capture in range(1, _lib.STREAM_SLOTS):  # from the middle on the slots are taken
         counters.update({16: capture, 32: capture})  # the same streams captured again, one forked to
-        held = [_lib.stream_tickets(cpu, s) for s in (16, 32)]
-        keep = list(_lib._local.counters.values())  # the graph's memory
-        assert held == [_lib.stream_tickets(cpu, s) for s in (16, 32)]
-        assert len(seen | set(held)) == len(seen) + 2
+        held = [_lib.stream_tickets(CPU, s) for s in (16, 32)]
+        assert held == [_lib.stream_tickets(CPU, s) for s in (16, 32)] and held[0] != held[1]
+        for a in held:
+            assert not in_slots(a) or a not in seen
+        if capture < _lib.STREAM_SLOTS // 2 - 1:
+            assert in_slots(held[0]) and in_slots(held[1])
         seen |= set(held)
         counters.clear()
-        assert _lib.stream_tickets(cpu, 16) == eager and not _lib._local.counters
-        assert all(int(buf.abs().sum()) == 0 for buf in keep)
+        assert _lib.stream_tickets(CPU, 16) == eager
+    assert not in_slots(held[1]) and not _lib._stream_tickets[0][0].any()
 
 
-def test_a_capture_makes_no_counters_for_eager_calls(counters):
-    """The first sliced call of a device may be a captured one; the eager calls' counters are made, and
-    zeroed, by an eager call."""
-    cpu = torch.device("cpu", 0)
-    counters[16] = 7
-    _lib.stream_tickets(cpu, 16)
-    assert not _lib._stream_tickets
+def test_counters_outside_the_slots_are_the_captures_own(counters):
+    """The first sliced call of a device may be a captured one: the slots are made, and zeroed, by an eager
+    call, the captured calls' counters are zeroed in their capture and go with it."""
+    held = []
+    for capture in (7, 8):
+        counters.update({16: capture, 32: capture})
+        at = [_lib.stream_tickets(CPU, s) for s in (16, 32, 16, 32)]
+        assert at[:2] == at[2:] and at[0] != at[1] and not _lib._stream_tickets
+        held.append(list(_lib._local.counters.values()))
+        assert [b.data_ptr() for b in held[-1]] == at[:2] and not any(b.any() for b in held[-1])
+    assert len({b.data_ptr() for bufs in held for b in bufs}) == 4
     counters.clear()
-    _lib.stream_tickets(cpu, 16)
-    assert len(_lib._stream_tickets) == 1
+    assert in_slots(_lib.stream_tickets(CPU, 16)) and not _lib._stream_tickets[0][0].any()
+    _lib.stream_tickets(CPU, 16, 9496)
+    assert _lib._local.capture == 0 and all(b is not h for b in _lib._local.counters.values() for h in held[-1])
 
 
 def test_streams_past_the_slots_share_none(counters):
-    """Each stream counts apart from the 64 that hold a slot, and from its neighbours, also past them."""
-    cpu = torch.device("cpu", 0)
-    at = [_lib.stream_tickets(cpu, 16 * s) for s in range(1, _lib.STREAM_SLOTS + 9)]
+    """Each stream counts apart from those that hold a slot, and from every other, also past them."""
+    streams = [16 * s for s in range(1, _lib.STREAM_SLOTS + 9)]
+    at = [_lib.stream_tickets(CPU, s) for s in streams]
     base = _lib._stream_tickets[0][0].data_ptr()
-    size = 4 * _lib.STREAM_TICKETS
-    assert sorted(at[:_lib.STREAM_SLOTS]) == [base + size * i for i in range(_lib.STREAM_SLOTS)]
-    assert all(not base <= a < base + size * _lib.STREAM_SLOTS for a in at[_lib.STREAM_SLOTS:])
-    assert all(a != b for a, b in zip(at[_lib.STREAM_SLOTS:], at[_lib.STREAM_SLOTS + 1:]))
+    assert sorted(at[:_lib.STREAM_SLOTS]) == [base + SIZE * i for i in range(_lib.STREAM_SLOTS)]
+    assert len(set(at)) == len(at) and not any(in_slots(a) for a in at[_lib.STREAM_SLOTS:])
     assert len(_lib._stream_tickets[0][1]) == _lib.STREAM_SLOTS
-    assert at[:_lib.STREAM_SLOTS] == [_lib.stream_tickets(cpu, 16 * s) for s in range(1, _lib.STREAM_SLOTS + 1)]
+    assert at == [_lib.stream_tickets(CPU, s) for s in streams]
+    for s in range(1, 200):  # what lies outside the slots stays bounded
+        _lib.stream_tickets(CPU, 16 * (s + 2 * _lib.STREAM_SLOTS))
+    assert len(_lib._local.counters) <= 65
 
 
 def test_the_other_kernels_calls_count_apart_too(counters, monkeypatch):
     """tickets() of the decode and skinny kernels: by stream, a capture's own, more of them when asked."""
-    cpu = torch.device("cpu", 0)
-
     def at(stream, count=160):
         monkeypatch.setattr(_lib, "stream", lambda device: stream)
-        buf = _lib.tickets(cpu, count)
-        assert buf.numel() >= count and not buf.any()
-        return buf
+        return _lib.tickets(CPU, count)
 
-    eager = [at(16 * s) for s in range(1, _lib.STREAM_SLOTS + 4)]
-    assert len({b.data_ptr() for b in eager}) == len(eager) and len(_lib._tickets) == _lib.STREAM_SLOTS
-    assert at(16) is eager[0] and at(16, 9496) is at(16, 9496) is not eager[0]
+    assert at(16) == at(16) == _lib.stream_tickets(CPU, 16) != at(32)
+    wide = at(16, 9496)
+    assert wide == at(16, 9496) and not in_slots(wide) and wide != at(32, 9496)
+    assert _lib._local.counters[0, 16].numel() >= 9496
+    eager = [at(16), at(32), wide]
     counters.update({16: 3, 32: 3})
-    held = [at(16), at(32), at(16)]
-    assert held[0] is held[2] is not held[1] and all(b is not h for b in _lib._tickets.values() for h in held)
+    held = [at(16), at(32), at(16, 9496)]
+    assert not set(held) & set(eager) and len(set(held)) == 3
     counters.update({16: 4})
-    assert at(16) is not held[0]
+    assert at(16) not in held
