@@ -121,8 +121,10 @@ def test_the_other_kernels_calls_count_apart_too(counters, monkeypatch):
     assert wide == at(16, 9496) and not in_slots(wide) and wide != at(32, 9496)
     assert _lib._local.counters[0, 16].numel() >= 9496
     eager = [at(16), at(32), wide]
+    keep = list(_lib._local.counters.values())
     counters.update({16: 3, 32: 3})
     held = [at(16), at(32), at(16, 9496)]
     assert not set(held) & set(eager) and len(set(held)) == 3
+    keep += _lib._local.counters.values()
     counters.update({16: 4})
-    assert at(16) not in held
+    assert at(16) not in held and at(16, 9496) not in held and not any(b.any() for b in keep)
