@@ -35,11 +35,10 @@ struct ResidentArgs {
   const void* x;
   const float* xs;  // FP8: token scales
   uint16_t* y;
-  float* sum;  // the fp32 output of QLX_MODE_SUM in several slices
   float* work;
   int* tickets;
   int m, n, k, half, swiglu;
-  int planes;         // the outputs are fp32 planes (K slices, or the planes themselves)
+  int planes;         // the outputs are fp32 planes (K slices, or the planes themselves); 2: y is their fp32 sum
   int units, per_slice, splits;
   int ntiles, groups, tblocks;
   int strided;        // a workgroup's tiles lie `groups` apart (whole K only)
@@ -500,8 +499,8 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) r
       const size_t o = (size_t)(m0 + mm) * a.half + row;
       store_pair(a.y, o, swiglu_bf(gv[0], uv[0]), swiglu_bf(gv[1], uv[1]));
       store_pair(a.y, o + 2, swiglu_bf(gv[2], uv[2]), swiglu_bf(gv[3], uv[3]));
-    } else if (a.sum) {
-      *gmem(reinterpret_cast<f32x4*>(a.sum + (size_t)(m0 + mm) * a.n + row)) = gv;
+    } else if (a.planes == 2) {
+      *gmem(reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.y) + (size_t)(m0 + mm) * a.n + row)) = gv;
     } else {
       const size_t o = (size_t)(m0 + mm) * a.n + row;
       store_pair(a.y, o, gv[0], gv[1]);
@@ -618,9 +617,8 @@ int resident_run(const char* name, ResidentArgs a, int m, int n, int k, const ql
   a.strided = p.splits == 1 && a.run >= 12;
   a.wbytes = (unsigned)((long long)(n / 16) * units * 1024);
   a.sbytes = (unsigned)((long long)n * (Unit<F>::NG ? units * Unit<F>::NG : 1) * 2);
-  a.planes = planes || sum || p.splits > 1;
-  a.sum = sum ? reinterpret_cast<float*>(a.y) : nullptr;
-  a.work = sum && p.splits == 1 ? a.sum : plan->workspace, a.tickets = !planes && p.splits > 1 ? plan->tickets : nullptr;
+  a.planes = sum ? 2 : planes || p.splits > 1;
+  a.work = sum && p.splits == 1 ? reinterpret_cast<float*>(a.y) : plan->workspace, a.tickets = !planes && p.splits > 1 ? plan->tickets : nullptr;
   const hipError_t e = m <= 16 ? resident_units<F, 1>(a, p.u, (hipStream_t)stream)
                                : resident_units<F, 2>(a, p.u, (hipStream_t)stream);
   return hip_status(e, name);
