@@ -193,6 +193,14 @@ __device__ __forceinline__ void unit_order(uint4 (&f)[Unit<F>::NF]) {
   }
 }
 
+// Orders the wave's LDS accesses across its lanes, which no barrier of the workgroup does here: the
+// hardware keeps a wave's LDS operations in order, this keeps the compiler from moving them (no instruction).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The code is kept small, one copy of each part: a launch of ~10 us runs it from a cold instruction
 // cache. (A first version, with the epilogue inlined per tile in flight and token fragment, had 31
 // to 138 KB of code and took 13.1 us where this one, 10 KB, takes 9.6: W4A16 gate_up of one token.)
@@ -345,10 +353,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) r
           const int row = t * ROWS + lane / CH;
           turn[row * CH + ((lane % CH) ^ (row / (16 / CH)))] = xf[u][mt][t];
         }
+        wave_lds_order();
         const int row = FEW ? r % ROWS : r;  // rows past the tokens: others', whose products are dropped
 #pragma unroll
         for (int t = 0; t < NF; ++t)
           xf[u][mt][t] = turn[row * CH + (frag_chunk<F>(c, t) ^ (row / (16 / CH)))];
+        wave_lds_order();
         if constexpr (!FP8) {
           unit_order<F>(xf[u][mt]);
 #pragma unroll
