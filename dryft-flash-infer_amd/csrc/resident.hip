@@ -29,18 +29,34 @@ int resident_splits(int m, int n, int k) {
   return best;
 }
 
-// Where another kernel streams a call faster, although this one serves it (us per call over distinct
-// weights, the other kernel / this one, MI355X). 8-bit weights of over 64 MiB, where both are at the
-// memory's rate and the other kernels' 8 waves of whole tiles read it more evenly: 151936 x 2560 FP8
-// 67.7 / 74.2 at one token, 72.3 / 78.2 at 8, 68.8 / 81.6 at 16, 102.7 / 113.5 at 64; W8A16 71.3 /
-// 71.5, 72.4 / 75.7, 67.8 / 81.2 (but 123.8 / 114.6 at 64). 4-bit weights of long runs at up to 4
-// tokens, where the ring kernel does (gemm.h): W4A16 37.5 / 38.9 at one token, 40.4 / 42.3 at 4,
-// 46.7 / 42.6 at 8. FP8 of one token: the other kernel quantizes it itself, one launch fewer.
-static bool resident_yields(int fmt, int m, int n, int k) {
+// Where another kernel streams a call faster, although this one serves it in `s` slices: the decode kernel
+// up to 8 tokens, the skinny GEMM above. The lines are measured: both kernels at 8643 calls of 1 to 64
+// tokens (n 1024 to 151936, k 1024 to 13824, distinct weights; MI355X), and at 1944 with SwiGLU; in
+// brackets this kernel's time over the other's past the line (geometric mean). What they
+// share is a workgroup's long run: probably as the other kernels' staging of the activation, which this one
+// saves, is then spread over many tiles, while its sums over 8 waves, and planes, are paid for each.
+// us per call, the other kernel / this one: 151936 x 2560 FP8 67.7 / 74.2 at one token, 68.8 / 81.6 at 16,
+// W8A16 72.4 / 75.7 at 8, 67.8 / 81.2 at 16 (but 123.8 / 114.6 at 64), W4A16 37.5 / 38.9 at one token,
+// 46.7 / 42.6 at 8; FP8 19456 x 2560 15.8 / 18.0 at 32; W8A16 32000 x 5120 52.7 / 61.1 at 64. FP8 of one
+// token takes a launch fewer there: that kernel quantizes it itself.
+static bool resident_yields(int fmt, int m, int n, int k, int s) {
   const long long bytes = (long long)n * k;
-  if (fmt == QLX_FMT_FP8) return m == 1 || bytes > (64ll << 20);
-  if (fmt == QLX_FMT_W8A16) return m <= 32 && bytes > (64ll << 20);
-  if (fmt == QLX_FMT_W4A16) return m <= 4 && n / 16 >= 2 * 8 * 256;
+  const int tiles = n / 16;
+  switch (fmt) {
+    case QLX_FMT_FP8:
+      if (m == 1 || bytes > (64ll << 20)) return true;
+      if (m >= 9) return tiles >= 1024 || (s > 1 && tiles >= 640);  // [1.06 to 32 tokens, 1.14 above]
+      return s > 1 && tiles >= (m <= 4 ? 256 : 512);                // [1.06, 1.08]
+    case QLX_FMT_W8A16:
+      if (m <= 32 && bytes > (64ll << 20)) return true;
+      if (m >= 33) return (s > 1 || k <= 1024) && tiles > 1792;  // [1.14]
+      return m >= 9 && tiles > (m <= 16 ? 1024 : 1536);          // [1.06, 1.06]
+    case QLX_FMT_W4A16:
+      if (m <= 4 && tiles >= 2 * 8 * 256) return true;
+      // 28672 x 2560 of 16 tokens 11.5 / 14.1, but 49152 x 2560 18.9 / 17.9
+      if (m >= 9 && m <= 32) return (tiles > 1536 && tiles <= 2048) || (m > 16 && s > 1 && tiles >= 4096);  // [1.05]
+      return m <= 2 && s > 1 && tiles >= 256 && tiles <= 512;  // [1.04]
+  }
   return false;
 }
 
@@ -73,7 +89,7 @@ int qlx_plan_resident(int fmt, int mode, int m, int n, int k, qlx_plan* plan) {
   p.waves = 8;
   p.kw = 8;
   p.rw = 1;
-  p.splits = resident_yields(fmt, m, n, k) ? 0 : s;
+  p.splits = resident_yields(fmt, m, n, k, s) ? 0 : s;
   *plan = p;
   return QLX_OK;
 }

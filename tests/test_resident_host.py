@@ -128,3 +128,29 @@ def test_the_other_kernels_calls_count_apart_too(counters, monkeypatch):
     keep += _lib._local.counters.values()
     counters.update({16: 4})
     assert at(16) not in held and at(16, 9496) not in held and not any(b.any() for b in keep)
+
+
+@pytest.mark.parametrize("name,n,k,ours,others", [
+    # 8-bit weights over 64 MiB, and FP8 of one token
+    ("fp8", 151936, 2560, (), (1, 2, 8, 16, 64)), ("w8a16", 151936, 2560, (33, 64), (1, 8, 16, 32)),
+    # long runs: from 1024 tiles (FP8), past 1024 and 1536 (W8A16), between 1536 and 2048 (W4A16)
+    ("fp8", 16368, 2560, (2, 8, 9, 32, 64), (1,)), ("fp8", 16384, 2560, (2, 8), (9, 16, 32, 33, 64)),
+    ("w8a16", 16384, 2560, (1, 8, 9, 16, 17, 64), ()), ("w8a16", 16400, 2560, (1, 8, 17, 32, 64), (9, 16)),
+    ("w8a16", 24576, 2048, (8, 17, 32, 33), (9, 16)), ("w8a16", 24592, 2048, (8, 33, 64), (9, 16, 17, 32)),
+    ("w4a16", 24576, 2560, (1, 8, 9, 16, 32, 64), ()), ("w4a16", 24592, 2560, (1, 8, 33, 64), (9, 16, 17, 32)),
+    ("w4a16", 32768, 2560, (1, 8, 33, 64), (9, 16, 17, 32)), ("w4a16", 32784, 2560, (1, 8, 9, 16, 32, 64), ()),
+    ("w4a16", 65520, 2560, (1, 4, 9, 32), ()), ("w4a16", 65536, 2560, (5, 8, 9, 32, 64), (1, 4)),
+    # runs of K slices
+    ("fp8", 4080, 8192, (2, 4, 8), (1,)), ("fp8", 4096, 8192, (8,), (2, 4)), ("fp8", 8192, 8192, (), (2, 4, 8)),
+    ("fp8", 10224, 6144, (9, 64), ()), ("fp8", 10240, 6144, (), (9, 16, 64)),
+    ("w8a16", 28672, 5120, (33, 64), ()), ("w8a16", 28688, 5120, (), (33, 64)), ("w8a16", 28688, 2560, (33, 64), ()),
+    ("w8a16", 28688, 1024, (), (33, 64)), ("w4a16", 65536, 5120, (16, 33), (17, 32)),
+    ("w4a16", 4096, 9728, (4,), (1, 2)), ("w4a16", 8208, 9728, (1, 2, 4), ()),
+    # the reference's formats, whose calls the decode kernel takes otherwise
+    ("int8g64", 151936, 2560, (1, 8, 16, 64), ()), ("int4g64", 151936, 2560, (1, 8, 16, 64), ())])
+def test_plan_leaves_the_calls_that_another_kernel_streams_faster(name, n, k, ours, others):
+    """Both sides of each line of the dispatch."""
+    for m in ours:
+        assert planned(FORMATS[name][0], m, n, k).splits >= 1, (name, n, k, m)
+    for m in others:
+        assert planned(FORMATS[name][0], m, n, k).splits == 0, (name, n, k, m)
