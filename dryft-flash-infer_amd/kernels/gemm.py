@@ -88,6 +88,7 @@ def _reference_candidates(batch, packed, quick):
 
 
 def _north_candidates(batch, packed, quick):
+    from . import qlinear
     tiles = getattr(packed[0], "tiles", packed[0])
     fmt = tiles.fmt
     bits = 4 if fmt == "w4a16" else 8
@@ -96,7 +97,9 @@ def _north_candidates(batch, packed, quick):
         lib_fmt = {"w8a16": _lib.FMT_W8A16, "w4a16": _lib.FMT_W4A16, "fp8": _lib.FMT_FP8}[fmt]
         plan = _linear.make_plan(lib_fmt, _lib.MODE_BF16, batch, tiles.rows, tiles.k)
         steps = tiles.k // (256 if fmt == "w4a16" else 128)
-        variants.append(("resident GEMM", {"resident": True}))
+        if (qlinear.aligned(tiles.weight, tiles.scale)
+                and qlinear.plan_resident(lib_fmt, batch, tiles.rows, tiles.k) is not None):
+            variants.append(("resident GEMM", {"resident": True}))
         for mul in (2, 4):
             if plan.splits * mul <= steps:
                 variants.append((f"decode split-K {plan.splits * mul}",

@@ -7,7 +7,7 @@ import types
 import pytest
 import torch
 
-from kernels import _lib
+from kernels import _lib, qlinear
 
 FORMATS = {"w4a16": (_lib.FMT_W4A16, 2), "w8a16": (_lib.FMT_W8A16, 1), "fp8": (_lib.FMT_FP8, 1),
            "int8g64": (_lib.FMT_REF8, 1), "int4g64": (_lib.FMT_REF4, 2)}  # format, codes a byte
@@ -154,3 +154,14 @@ def test_plan_leaves_the_calls_that_another_kernel_streams_faster(name, n, k, ou
         assert planned(FORMATS[name][0], m, n, k).splits >= 1, (name, n, k, m)
     for m in others:
         assert planned(FORMATS[name][0], m, n, k).splits == 0, (name, n, k, m)
+
+
+@pytest.mark.parametrize("fmt,m,has", [("fp8", 1, False), ("fp8", 8, True), ("w8a16", 1, True), ("w4a16", 64, True)])
+def test_a_race_has_the_resident_gemm_where_its_plan_has_the_call(fmt, m, has):
+    """A candidate named for a kernel is that kernel, not what serves the call without it."""
+    from kernels import gemm
+    weight = torch.zeros(2560, 512 if fmt == "w4a16" else 1024, dtype=torch.uint8)
+    tiles = qlinear.Tiled(weight, torch.zeros(2560 * (8 if fmt == "w4a16" else 1), dtype=torch.bfloat16), 2560, 1024, fmt)
+    assert has == any("resident" in c.label for c in gemm._north_candidates(m, [tiles], False))
+    off = qlinear.Tiled(torch.zeros(weight.numel() + 8, dtype=torch.uint8)[8:], tiles.scale, 2560, 1024, fmt)
+    assert off.weight.data_ptr() % 16 and not any("resident" in c.label for c in gemm._north_candidates(m, [off], False))
