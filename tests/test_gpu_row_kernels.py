@@ -75,12 +75,23 @@ def test_quantize_fp8_activation_widths(k):
     assert np.array_equal(q.view(torch.uint8).cpu().numpy(), q0) and np.array_equal(s.cpu().numpy(), s0)
 
 
+def int8_heads(bits):
+    """Codes and scales of bf16 heads as the kernel forms them: a NaN counts in no maximum and takes the code
+    -127, as does an infinity over the infinite scale it makes, under which finite values take 0."""
+    y = O.bf16_to_f32(bits)
+    amax = np.where(np.isnan(y), np.float32(0), np.abs(y)).max(-1)
+    scale = (np.maximum(amax, np.float32(1e-12)) / np.float32(127)).astype(np.float32)
+    with np.errstate(invalid="ignore"):
+        code = np.floor((y / scale[..., None]).astype(np.float32) + np.float32(0.5))
+    return np.where(np.isnan(code), -127, np.clip(code, -127, 127)).astype(np.int8), scale
+
+
 @pytest.mark.parametrize("n_q,n_kv", [(1, 1), (5, 3), (32, 8), (3, 0), (40, 10)])
 @pytest.mark.parametrize("int8", [False, True])
 @pytest.mark.parametrize("special", [False, True])
 def test_rope_head_counts(n_q, n_kv, int8, special):
-    """Heads share 16-lane groups and waves across the Q / K / V boundaries; a head of zeros, of a NaN
-    and (INT8) of infinities."""
+    """Heads share 16-lane groups and waves across the Q / K / V boundaries; a head of zeros; value and key
+    heads with a NaN and with infinities, whose INT8 codes the oracle leaves open (int8_heads)."""
     print("rope", n_q, n_kv, int8, special, flush=True)
     rows, cap, pos = 3, 20, 17
     qkv = rand(rows, (n_q + 2 * n_kv) * 128, seed=n_q)
@@ -88,16 +99,20 @@ def test_rope_head_counts(n_q, n_kv, int8, special):
     if special:
         qkv[1, 3] = float("nan")
         qkv[1, -5] = float("nan")
-        qkv[2, -9] = float("inf")
+        qkv[2, -9], qkv[2, -77] = float("inf"), float("-inf")
+        if n_kv:
+            qkv[0, n_q * 128 + 7] = float("inf")
+            qkv[1, n_q * 128 + 70] = float("nan")
     qn, kn = rand(128, seed=1), rand(128, seed=2)
     ang = torch.randn(cap, 128, generator=torch.Generator().manual_seed(9))
     cos, sin = ang.cos().to(torch.bfloat16), ang.sin().to(torch.bfloat16)
     kv = max(n_kv, 1)
     kc = np.zeros((rows, kv, cap, 128), np.int8 if int8 else np.uint16)
     vc, ks, vs = kc.copy(), np.zeros((rows, kv, cap), np.float32), np.zeros((rows, kv, cap), np.float32)
+    kw, vw = (np.zeros((rows, kv, 1, 128), np.uint16) for _ in range(2))
     with np.errstate(invalid="ignore", over="ignore"):
         q0 = A.qkv_norm_rope_to_cache(bits16(qkv), n_q, n_kv, bits16(qn), bits16(kn), bits16(cos), bits16(sin), [pos], 1, kc,
-                                      vc, 1e-6, *((ks, vs) if int8 else ()))
+                                      vc, 1e-6, *((ks, vs) if int8 else (None, None)), kw, vw)
     if n_kv == 0:
         from kernels import q_norm_rope
         got = q_norm_rope(qkv.to(DEV), n_q, qn.to(DEV), cos.to(DEV), sin.to(DEV),
@@ -110,13 +125,13 @@ def test_rope_head_counts(n_q, n_kv, int8, special):
                                  torch.tensor([pos], dtype=torch.int32, device=DEV), 1, kd, vd, 1e-6, ksd, vsd)
     same(got, q0)
     if int8:
-        bad = ~np.isfinite(ks[..., pos]) | ~np.isfinite(vs[..., pos])
-        if special:  # a head holding a NaN: its code is -127 here, unspecified in the oracle
-            bad[1, -1] = True
-            bad[1, 0] |= n_q == 0
-        ok = ~bad
-        assert np.array_equal(kd.cpu().numpy()[ok], kc[ok]) and np.array_equal(vd.cpu().numpy()[ok], vc[ok])
-        assert np.array_equal(ksd.cpu().numpy()[ok], ks[ok]) and np.array_equal(vsd.cpu().numpy()[ok], vs[ok])
+        for codes, scales, cache, factors, heads in ((kd, ksd, kc, ks, kw), (vd, vsd, vc, vs, vw)):
+            want, factor = int8_heads(heads[:, :, 0])
+            ok = ((heads[:, :, 0] & 0x7FFF) < 0x7F80).all(-1)
+            assert ok.all() != special
+            assert np.array_equal(want[ok], cache[:, :, pos][ok]) and np.array_equal(factor[ok], factors[..., pos][ok])
+            assert np.array_equal(codes.cpu().numpy()[:, :, pos], want) and np.array_equal(scales.cpu().numpy()[..., pos], factor)
+            assert not codes.cpu().numpy()[:, :, :pos].any() and not codes.cpu().numpy()[:, :, pos + 1:].any()
     else:
         same(kd, kc)
         same(vd, vc)
