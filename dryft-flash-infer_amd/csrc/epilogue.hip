@@ -35,10 +35,6 @@ residual_planes_kernel(const uint16_t* __restrict__ x, const float* __restrict__
   out[i] = f2bf(bf2f(x[i]) + round_bf(acc));
 }
 
-__device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
-  return (uint32_t)f2bf(lo) | ((uint32_t)f2bf(hi) << 16);
-}
-
 __device__ __forceinline__ uint4 ld16(const uint16_t* p) {
   const u32x4 v = *gmem(reinterpret_cast<const u32x4*>(p));
   return uint4{v[0], v[1], v[2], v[3]};

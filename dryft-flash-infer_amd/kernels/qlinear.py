@@ -198,7 +198,8 @@ def _skinny(fmt, q, s, x, n, k, swiglu, fused_reduce=None):
 
 #: Up to this many tokens the resident-activation GEMM (``qlx_linear_resident``) is the default where
 #: its plan has the call; ``resident=True`` takes it at any batch. From 9 tokens these functions'
-#: default stays the skinny GEMM, whose bits callers compare with ``qlx_linear_skinny``'s; the
+#: default stays the skinny GEMM, so that their results are ``qlx_linear_skinny``'s bit for bit, also
+#: where the resident GEMM is faster (W4A16 gate_up and down of 64 tokens 36.9 us, 32.4 with it); the
 #: engine's call sites (``cuda_fp8.matmul``, ``gate_up_swiglu``) pass ``resident=True``.
 RESIDENT_TO = 8
 
