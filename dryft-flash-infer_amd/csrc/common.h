@@ -44,8 +44,9 @@ __device__ __forceinline__ float round_bf(float f) { return bf2f(f2bf(f)); }
 // Two fp32 values to a bf16 pair (lo in the low half) by the hardware's round-to-nearest-even
 // conversion (v_cvt_pk_bf16_f32): the same bits as f2bf for every value but a NaN (checked on
 // MI355X over all 2^32 inputs; a NaN keeps its payload's top bits instead of becoming
-// sign | 0x7FC0). Where a NaN's bits are a result they go through bf16_canonical_nan (the
-// executor's stages redo the chunk with f2bf); where the pair only feeds further arithmetic (attention's dequantized cache, SwiGLU's inputs) any NaN does.
+// sign | 0x7FC0). Where a NaN's bits are a result they go through bf16_canonical_nan (the executor's
+// stages redo the chunk with f2bf); where the pair only feeds further arithmetic (attention's
+// dequantized cache, SwiGLU's inputs) any NaN does.
 __device__ __forceinline__ uint32_t bf16_pair_hw(float lo, float hi) {
   typedef __attribute__((ext_vector_type(2))) float f2;
   typedef __attribute__((ext_vector_type(2))) __bf16 b2;
