@@ -137,35 +137,47 @@ struct Fp8Quant {
 // (IEEE division, ~30 instructions a value, and the values read twice): 151936 x 2560 to int4 in
 // 1362 us, 0.7 TB/s. Groups of up to 512 values: L lanes (8 values each) per group, 4 groups per
 // thread loaded before any is reduced: the same weight in 221 us, 4.4 TB/s (a large copy: 4.9 TB/s).
-constexpr int kSegs = 4;
-template <class Q, int L>
+// Groups of 513 to 2048 values: 2 or 4 chunks a lane of a whole wave. (A block per group leaves half of its
+// lanes without values: 40960 x 2048 to e4m3 in groups of 1024 68.8 us, a wave that reads the group twice
+// 47.1, this 40.7; 40960 x 2080 in groups of 520 129.5, 79.1 and 57.1.)
+template <class Q, int L, int CHUNKS = 1>
 __global__ void __launch_bounds__(256)
 quantize_segments_kernel(Q quant, const uint16_t* __restrict__ w, void* __restrict__ data,
                          uint16_t* __restrict__ scale, long long segs, int group) {
   const int lane = threadIdx.x % L, octets = group >> 3;
-  constexpr int PER = 256 / L;
-  const long long seg0 = (long long)blockIdx.x * (PER * kSegs) + threadIdx.x / L;
-  uint4 v[kSegs];
+  constexpr int PER = 256 / L, SEGS = 4 / CHUNKS;
+  const long long seg0 = (long long)blockIdx.x * (PER * SEGS) + threadIdx.x / L;
+  uint4 v[SEGS][CHUNKS];
 #pragma unroll
-  for (int u = 0; u < kSegs; ++u) {
+  for (int u = 0; u < SEGS; ++u) {
     const long long seg = seg0 + u * PER;
-    v[u] = uint4{0u, 0u, 0u, 0u};
-    if (seg < segs && lane < octets) v[u] = *reinterpret_cast<const uint4*>(w + (size_t)seg * group + 8 * lane);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int o = lane + L * c;
+      v[u][c] = uint4{0u, 0u, 0u, 0u};
+      if (seg < segs && o < octets) v[u][c] = *reinterpret_cast<const uint4*>(w + (size_t)seg * group + 8 * o);
+    }
   }
 #pragma unroll
-  for (int u = 0; u < kSegs; ++u) {
+  for (int u = 0; u < SEGS; ++u) {
     const long long seg = seg0 + u * PER;
-    float amax = octet_amax(v[u], 0.f);
+    float amax = 0.f;
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) amax = octet_amax(v[u][c], amax);
 #pragma unroll
     for (int o = L / 2; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
     if (seg >= segs) continue;
     const typename Q::Group g = quant.group(amax);
     if (lane == 0) scale[seg] = g.sbits;
-    if (lane < octets) quant.store(g, v[u], data, (size_t)seg * group + 8 * lane);
+#pragma unroll
+    for (int c = 0; c < CHUNKS; ++c) {
+      const int o = lane + L * c;
+      if (o < octets) quant.store(g, v[u][c], data, (size_t)seg * group + 8 * o);
+    }
   }
 }
 
-// Groups of 513 to 256 * 8 * R values (a row per scale): a 256-thread block per group, which keeps
+// Groups of 2049 to 256 * 8 * R values (a row per scale): a 256-thread block per group, which keeps
 // its values in registers between the maximum and the codes.
 template <class Q, int R>
 __global__ void __launch_bounds__(256)
@@ -219,14 +231,17 @@ void launch_quantize(const Q& quant, const uint16_t* w, void* data, uint16_t* sc
                      hipStream_t st) {
   const long long segs = (long long)rows * (k / group);
   const int octets = group >> 3;
-  auto segments = [&](auto lc) {
-    constexpr int L = decltype(lc)::value, per = 256 / L * kSegs;
-    quantize_segments_kernel<Q, L><<<(unsigned)((segs + per - 1) / per), 256, 0, st>>>(quant, w, data, scale, segs, group);
+  auto segments = [&](auto lc, auto cc) {
+    constexpr int L = decltype(lc)::value, C = decltype(cc)::value, per = 256 / L * (4 / C);
+    quantize_segments_kernel<Q, L, C><<<(unsigned)((segs + per - 1) / per), 256, 0, st>>>(quant, w, data, scale, segs, group);
   };
-  if (octets <= 8) segments(std::integral_constant<int, 8>{});
-  else if (octets <= 16) segments(std::integral_constant<int, 16>{});
-  else if (octets <= 32) segments(std::integral_constant<int, 32>{});
-  else if (octets <= 64) segments(std::integral_constant<int, 64>{});
+  constexpr std::integral_constant<int, 1> one{};
+  if (octets <= 8) segments(std::integral_constant<int, 8>{}, one);
+  else if (octets <= 16) segments(std::integral_constant<int, 16>{}, one);
+  else if (octets <= 32) segments(std::integral_constant<int, 32>{}, one);
+  else if (octets <= 64) segments(std::integral_constant<int, 64>{}, one);
+  else if (octets <= 128) segments(std::integral_constant<int, 64>{}, std::integral_constant<int, 2>{});
+  else if (octets <= 256) segments(std::integral_constant<int, 64>{}, std::integral_constant<int, 4>{});
   else if (octets <= 512) quantize_rows_kernel<Q, 2><<<(unsigned)segs, 256, 0, st>>>(quant, w, data, scale, group);
   else if (octets <= 2048) quantize_rows_kernel<Q, 8><<<(unsigned)segs, 256, 0, st>>>(quant, w, data, scale, group);
   else quantize_wave_kernel<Q><<<(unsigned)((segs + 3) / 4), 256, 0, st>>>(quant, w, data, scale, segs, group);

@@ -32,7 +32,7 @@ def weight(n, k, seed):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("k,group", [(24, 8), (120, 40), (192, 64), (576, 72), (384, 128), (400, 200), (1024, 512),
-                                     (1040, 520), (4096, 4096), (4104, 4104), (16384, 16384), (16392, 16392)])
+                                     (1040, 520), (1024, 1024), (1032, 1032), (4096, 2048), (2056, 2056), (4096, 4096), (4104, 4104), (16384, 16384), (16392, 16392)])
 @pytest.mark.parametrize("bits,scale,storage", [(8, "f16", "offset"), (8, "bf16", "signed"), (4, "f16", "offset"),
                                                 (4, "bf16", "k32")])
 def test_quantize_group_lengths(k, group, bits, scale, storage):
@@ -60,7 +60,8 @@ def test_quantize_group_lengths(k, group, bits, scale, storage):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("k,group", [(48, 8), (384, 128), (1040, 520), (9728, 9728), (16392, 16392)])
+@pytest.mark.parametrize("k,group", [(48, 8), (384, 128), (1040, 520), (2048, 1024), (1032, 1032), (2048, 2048), (2056, 2056),
+                                     (9728, 9728), (16392, 16392)])
 def test_quantize_fp8_group_lengths(k, group):
     print("quantize fp8", k, group, flush=True)
     w = weight(19, k, k)
