@@ -159,6 +159,17 @@ extern "C" int qlx_plan_fit(qlx_plan* plan, int fmt, int m, int n, int k, int co
   return QLX_OK;
 }
 
+// The K slices of a call that asks for `splits` on the planned workgroup shape: qlx_plan_linear, then
+// qlx_plan_fit with grow. Negative: a status.
+extern "C" int qlx_plan_slices(int fmt, int mode, int m, int n, int k, int splits) {
+  qlx_plan p;
+  int rc = qlx_plan_linear(fmt, mode, m, n, k, &p);
+  if (rc) return rc;
+  p.splits = splits;
+  rc = qlx_plan_fit(&p, fmt, m, n, k, 1, 1);
+  return rc ? rc : p.splits;
+}
+
 // The capture that a stream is in (0: none), the same for every stream that the capture has forked to.
 // A stream that the runtime refuses to query counts as not captured: the launch on it reports the error.
 extern "C" unsigned long long qlx_stream_capture(void* stream) {

@@ -103,6 +103,7 @@ SIGNATURES = {
     "qlx_plan_tickets": ([_PLAN, _I, _I, _I, _I], _I),
     "qlx_stream_capture": ([_P], ctypes.c_ulonglong),
     "qlx_plan_fit": ([_PLAN, _I, _I, _I, _I, _I, _I], _I),
+    "qlx_plan_slices": ([_I, _I, _I, _I, _I, _I], _I),
     "qlx_tile_rows": ([_P, _P, _I, _I, _P], _I),
     "qlx_linear_w8a16": ([_P, _P, _P, _P, _I, _I, _I, _I, _PLAN, _P], _I),
     "qlx_linear_w4a16": ([_P, _P, _P, _P, _I, _I, _I, _I, _PLAN, _P], _I),

@@ -263,8 +263,7 @@ def _resident_plan(prepared, batch, config, mode):
         return None
     plan = qlinear.plan_resident(fmt, batch, prepared.rows, prepared.k, mode == _lib.MODE_SWIGLU)
     if plan is not None and mode == _lib.MODE_PLANES:
-        cfg = _plan_config(prepared, batch, config, mode)
-        one = _linear.splits_for(fmt, mode, batch, prepared.rows, prepared.k, cfg, fit=True) == 1
+        one = _lib.lib().qlx_plan_slices(fmt, mode, batch, prepared.rows, prepared.k, 1) == 1
         plan.mode = _lib.MODE_SUM if one else mode
     return plan
 

@@ -145,6 +145,9 @@ unsigned long long qlx_stream_capture(void* stream);
  * plan's LDS fits (the reference's _plan, engine/kernels/cuda_fp8.py:1255-1276). comp =
  * activation components (2 only for QLX_FMT_INT8 with a residual component). */
 int qlx_plan_fit(qlx_plan* plan, int fmt, int m, int n, int k, int comp, int grow);
+/* The K slices that a call asking for `splits` takes on the workgroup shape of qlx_plan_linear (as
+ * qlx_plan_fit with grow); negative: a QLX_E* status. */
+int qlx_plan_slices(int fmt, int mode, int m, int n, int k, int splits);
 
 /* W8A16 per output channel. Replaces the W8A16 call of cuda_fp8.matmul
  * (engine/kernels/cuda_fp8.py:1316-1330) for the north-star per-channel format. */

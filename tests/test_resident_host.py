@@ -165,3 +165,16 @@ def test_a_race_has_the_resident_gemm_where_its_plan_has_the_call(fmt, m, has):
     assert has == any("resident" in c.label for c in gemm._north_candidates(m, [tiles], False))
     off = qlinear.Tiled(torch.zeros(weight.numel() + 8, dtype=torch.uint8)[8:], tiles.scale, 2560, 1024, fmt)
     assert off.weight.data_ptr() % 16 and not any("resident" in c.label for c in gemm._north_candidates(m, [off], False))
+
+
+def test_plan_slices_is_the_planned_shape_fitted():
+    """qlx_plan_slices: what make_plan and a fit of its workgroup shape give in turn."""
+    from kernels import _linear
+    for fmt in (_lib.FMT_REF8, _lib.FMT_REF4, _lib.FMT_W8A16):
+        for n, k in ((512, 1024), (2560, 9728), (19456, 2560), (4096, 28672)):
+            for m in (1, 8, 17, 64):
+                for ask in (1, 4):
+                    base = _linear.make_plan(fmt, _lib.MODE_PLANES, m, n, k)
+                    want = _linear.splits_for(fmt, _lib.MODE_PLANES, m, n, k, (base.waves, base.kw, base.rw, ask), fit=True)
+                    assert _lib.lib().qlx_plan_slices(fmt, _lib.MODE_PLANES, m, n, k, ask) == want
+    assert _lib.lib().qlx_plan_slices(_lib.FMT_REF8, 0, 0, 512, 1024, 1) == _lib.QLX_EINVAL
