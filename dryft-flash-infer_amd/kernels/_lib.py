@@ -236,6 +236,8 @@ def stream_tickets(device, stream, count=STREAM_TICKETS):
     capture their zeroing would be a node of that graph. Counters zeroed in a capture cost its replays
     that node, 1 to 4 us."""
     capture = capture_id(stream)
+    if _local.capture != capture:  # an ended capture's go back to its pool
+        _local.capture, _local.counters = capture, {}
     index = device.index if device.index is not None else torch.cuda.current_device()
     pool = _stream_tickets.get(index)
     if pool is None and not capture:
@@ -249,10 +251,10 @@ def stream_tickets(device, stream, count=STREAM_TICKETS):
             slot = slots.setdefault((stream, capture), next(numbers))
         if slot is not None and slot < STREAM_SLOTS:
             return buf.data_ptr() + slot * STREAM_TICKETS * 4
-    if _local.capture != capture or len(_local.counters) > 64:
-        _local.capture, _local.counters = capture, {}
     buf = _local.counters.get((index, stream))
     if buf is None or buf.numel() < count:
+        if len(_local.counters) >= 64:
+            _local.counters = {}
         buf = torch.zeros(max(count, STREAM_TICKETS), dtype=torch.int32, device=device)
         _local.counters[index, stream] = buf
     return buf.data_ptr()
